@@ -218,7 +218,12 @@ struct ActLayout {
 // Weight types with a tiled prefill GEMM (more than 16 activation columns);
 // the others run it as 16-column slabs of the few-column kernel.
 __host__ __device__ constexpr bool has_gemm(int wtype) {
-    return wtype == TLH_TYPE_Q4_K || wtype == TLH_TYPE_Q5_K || wtype == TLH_TYPE_Q8_0 || wtype == TLH_TYPE_Q4_0;
+    return kquant_type(wtype) || wtype == TLH_TYPE_Q8_0 || wtype == TLH_TYPE_Q4_0;
+}
+// Which k-quant GEMM that is: the int8-plane one (gemm_kq.hip), or the f16 one
+// of q4_K / q5_K (gemm.hip).
+__host__ __device__ constexpr bool gemm_is_kq(int wtype) {
+    return kquant_type(wtype) && wtype != TLH_TYPE_Q4_K && wtype != TLH_TYPE_Q5_K;
 }
 // q4_K / q5_K GEMM launches also get the activation codes as f16.
 __host__ __device__ constexpr bool act_has_f16(int wtype, int64_t n_cols) {

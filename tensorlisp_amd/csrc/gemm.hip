@@ -31,9 +31,10 @@
 //
 // q5_K runs the same kernel with the fifth code bit OR-ed in before the f16
 // conversion (sc * q <= 63 * 31 stays exact). q8_0 / q4_0 have their own
-// int8-MFMA GEMM (gemm_q8.hip). q6_K weights with N > 16 run through the
-// int8-MFMA few-column kernel (gemv_mfma.hip) in slabs of 16 columns (correct
-// for any N; each slab re-reads the weights).
+// int8-MFMA GEMM (gemm_q8.hip), q2_K / q3_K / q6_K the int8-plane one
+// (gemm_kq.hip). The other types (q4_1, q5_0, q5_1) run through the int8-MFMA
+// few-column kernel (gemv_mfma.hip) in slabs of 16 columns (correct for any N;
+// each slab re-reads the weights).
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -417,6 +418,14 @@ static int gemm_nw(int64_t N) { return N > 128 ? 8 : 4; }
 int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
     if (!has_gemm(wtype) || N <= 16) return 1;
     constexpr int64_t CUS = 256;  // MI355X
+    if (gemm_is_kq(wtype)) {  // as many chunks as one round of workgroups holds, four super-blocks each at least
+        const KqTile t = gemm_kq_tile(N);
+        const int64_t tiles = (N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * batches, units = K / 256;
+        int64_t ks = CUS * t.per_cu / tiles;
+        if (ks > units / 4) ks = units / 4;
+        if (ks > 16) ks = 16;
+        return ks > 1 ? (int)ks : 1;
+    }
     // workgroups that fit the CUs at once: two 128 x 128 tiles a CU (q8_0 /
     // q4_0, and q4_K / q5_K up to 128 tokens), one 128 x 256 tile (q4_K / q5_K above)
     const bool wide = (wtype == TLH_TYPE_Q4_K || wtype == TLH_TYPE_Q5_K) && gemm_nw(N) == 8;
@@ -471,8 +480,8 @@ tlh_status launch_gemm(const MatmulArgs &a, hipStream_t stream) {
         const tlh_status st = launch_gemm_q8(a, ks, stream);
         return st != TLH_OK || ks == 1 || a.keep_part ? st : launch_partial_reduce(a, ks, stream);
     }
-    if (a.wtype == TLH_TYPE_Q4_K || a.wtype == TLH_TYPE_Q5_K) {
-        const tlh_status st = launch_gemm_q4k(a, ks, stream);
+    if (kquant_type(a.wtype)) {
+        const tlh_status st = gemm_is_kq(a.wtype) ? launch_gemm_kq(a, ks, stream) : launch_gemm_q4k(a, ks, stream);
         return st != TLH_OK || ks == 1 || a.keep_part ? st : launch_partial_reduce(a, ks, stream);
     }
     if (a.keep_part) return set_error(TLH_UNSUPPORTED, "gemm: no kept partials for weight type %d", a.wtype);

@@ -209,6 +209,12 @@ tlh_status launch_partial_reduce(const MatmulArgs &a, int chunks, hipStream_t st
 // reduce_epi_check: TLH_OK when it takes a and ep
 tlh_status launch_partial_reduce_epi(const MatmulArgs &a, int chunks, const GemvEpi &ep, hipStream_t stream);
 tlh_status reduce_epi_check(const MatmulArgs &a, const GemvEpi &ep);
+// Int8-plane GEMM for k-quant weights (gemm_kq.hip), any N; ksplit as above.
+tlh_status launch_gemm_kq(const MatmulArgs &a, int ksplit, hipStream_t stream);
+struct KqTile {
+    int bm, bn, per_cu;  // weight rows, tokens, workgroups a CU holds
+};
+KqTile gemm_kq_tile(int64_t N);
 // K chunks of the tiled prefill GEMMs: a launch of fewer 128 x 128 tiles than
 // CUs splits K into up to 512 / tiles chunks (whole stages per chunk, at least four super-blocks /
 // sixteen q8_0 blocks each), and the bytes of its partial sums.

@@ -796,8 +796,7 @@ bool tlh::mul_mat_partials(const tlh_op *op, MmPartials &pp) {
     if (check_mul_mat(op, s) != TLH_OK || mm_empty(s) || s.flt || s.ne12 * s.ne13 != 1 || s.N < 3) return false;
     int64_t chunks;
     if (s.N > 16) {
-        if (s.wtype != TLH_TYPE_Q8_0 && s.wtype != TLH_TYPE_Q4_0 && s.wtype != TLH_TYPE_Q4_K && s.wtype != TLH_TYPE_Q5_K)
-            return false;
+        if (!has_gemm(s.wtype)) return false;
         chunks = gemm_ksplit(s.wtype, s.M, s.N, s.K, 1);
     } else {
         chunks = gemv_mfma_chunks(s.K);  // (the tall form takes K <= 4096: one chunk)
