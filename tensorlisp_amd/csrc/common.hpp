@@ -198,21 +198,16 @@ template <int WT> __device__ __forceinline__ float dequant_elem(const uint8_t *r
 //   sum : int32 [R][K/32] (q8_0)  per-block code sums
 //         f32   [R][K/32] (q8_1)  per-block s (f16-rounded code sum * d, as f32)
 //         int16 [R][K/16] (q8_K)  bsums
-//   q16 : f16   [R][K]            (GEMM launches only) the codes as f16,
-//         exact, so the MFMA operand needs no conversion
-//   b16 : f16   [R][K/16]         (GEMM launches, q8_K only) the bsums as f16 (exact)
 struct ActView {
     const int8_t *qs;
     const float *d;
     const int32_t *sum32;  // q8_0: code sums; q8_1: the bits of s as f32
     const int16_t *bsums;  // q8_K only
-    const _Float16 *q16;   // GEMM launches only
-    const _Float16 *b16;   // GEMM launches, q8_K only
     int64_t K;
 };
 
 struct ActLayout {
-    int64_t qs_off, d_off, sum_off, q16_off, b16_off, total;
+    int64_t qs_off, d_off, sum_off, total;
 };
 
 // Weight types with a tiled prefill GEMM (more than 16 activation columns);
@@ -220,29 +215,17 @@ struct ActLayout {
 __host__ __device__ constexpr bool has_gemm(int wtype) {
     return kquant_type(wtype) || wtype == TLH_TYPE_Q8_0 || wtype == TLH_TYPE_Q4_0;
 }
-// Which k-quant GEMM that is: the int8-plane one (gemm_kq.hip), or the f16 one
-// of q4_K / q5_K (gemm.hip).
-__host__ __device__ constexpr bool gemm_is_kq(int wtype) {
-    return kquant_type(wtype) && wtype != TLH_TYPE_Q4_K && wtype != TLH_TYPE_Q5_K;
-}
-// q4_K / q5_K GEMM launches also get the activation codes as f16.
-__host__ __device__ constexpr bool act_has_f16(int wtype, int64_t n_cols) {
-    return (wtype == TLH_TYPE_Q4_K || wtype == TLH_TYPE_Q5_K) && n_cols > 16;
-}
 
 __host__ __device__ inline int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
-__host__ __device__ inline ActLayout act_layout(int act_type, int64_t K, int64_t rows, bool f16 = false) {
+__host__ __device__ inline ActLayout act_layout(int act_type, int64_t K, int64_t rows) {
     ActLayout L;
     L.qs_off = 0;
     L.d_off = align_up(rows * K, 256);
     const int64_t nblk = K / block_elems(act_type);
     L.sum_off = align_up(L.d_off + rows * nblk * 4, 256);
     const int64_t sum_bytes = act_type == TLH_TYPE_Q8_K ? rows * (K / 16) * 2 : rows * (K / 32) * 4;
-    L.q16_off = align_up(L.sum_off + sum_bytes, 256);
-    L.b16_off = align_up(L.q16_off + rows * K * 2, 256);
-    L.total = f16 ? align_up(L.b16_off + (act_type == TLH_TYPE_Q8_K ? rows * (K / 16) * 2 : 0), 256)
-                  : align_up(L.q16_off, 256);
+    L.total = align_up(L.sum_off + sum_bytes, 256);
     return L;
 }
 
@@ -254,8 +237,6 @@ __host__ __device__ inline ActView act_view(const void *base, int act_type, int6
     v.d = (const float *)(b + L.d_off);
     v.sum32 = (const int32_t *)(b + L.sum_off);
     v.bsums = (const int16_t *)(b + L.sum_off);
-    v.q16 = (const _Float16 *)(b + L.q16_off);
-    v.b16 = (const _Float16 *)(b + L.b16_off);
     v.K = K;
     return v;
 }
@@ -327,22 +308,10 @@ __device__ __forceinline__ void q8K_waves(const float (&v)[NB][4], int lane, uin
 // One q8_K block (q8K_waves' results) into the split layout at activation
 // row `orow`, super-block `blk`.
 __device__ __forceinline__ void q8K_store_split(char *out, const ActLayout &L, int64_t K, int64_t orow, int64_t blk,
-                                                int lane, uint32_t packed, int psum, float d, bool f16) {
+                                                int lane, uint32_t packed, int psum, float d) {
     const int64_t e0 = orow * K + blk * QKK + 4 * lane;
     *(uint32_t *)(out + L.qs_off + e0) = packed;
-    if (f16) {
-        uint32_t h[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int c0 = (int)(int8_t)(packed >> (16 * i)), c1 = (int)(int8_t)(packed >> (16 * i + 8));
-            h[i] = (uint32_t)f2h((float)c0) | ((uint32_t)f2h((float)c1) << 16);
-        }
-        *(uint2 *)(out + L.q16_off + e0 * 2) = make_uint2(h[0], h[1]);
-    }
-    if ((lane & 3) == 0) {
-        ((int16_t *)(out + L.sum_off))[orow * (K / 16) + blk * 16 + (lane >> 2)] = (int16_t)psum;
-        if (f16) ((uint16_t *)(out + L.b16_off))[orow * (K / 16) + blk * 16 + (lane >> 2)] = f2h((float)psum);
-    }
+    if ((lane & 3) == 0) ((int16_t *)(out + L.sum_off))[orow * (K / 16) + blk * 16 + (lane >> 2)] = (int16_t)psum;
     if (lane == 0) ((float *)(out + L.d_off))[orow * (K / QKK) + blk] = d;
 }
 
@@ -357,7 +326,7 @@ __device__ __forceinline__ void q8K_store_split(char *out, const ActLayout &L, i
 template <int NB, bool Q81>
 __device__ __forceinline__ void q80_quads_store_split(const float (&v)[NB][4], const bool (&live)[NB], int lane,
                                                       char *out, const ActLayout &L, int64_t K, int64_t orow,
-                                                      const int64_t (&col)[NB], bool f16) {
+                                                      const int64_t (&col)[NB]) {
 #pragma clang fp contract(off)
     float amax[NB];
 #pragma unroll
@@ -392,15 +361,6 @@ __device__ __forceinline__ void q80_quads_store_split(const float (&v)[NB][4], c
         if (!live[b]) continue;
         const int64_t e0 = orow * K + col[b];
         *(uint32_t *)(out + L.qs_off + e0) = packed[b];
-        if (f16) {
-            uint32_t h[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int c0 = (int)(int8_t)(packed[b] >> (16 * i)), c1 = (int)(int8_t)(packed[b] >> (16 * i + 8));
-                h[i] = (uint32_t)f2h((float)c0) | ((uint32_t)f2h((float)c1) << 16);
-            }
-            *(uint2 *)(out + L.q16_off + e0 * 2) = make_uint2(h[0], h[1]);
-        }
         if ((lane & 7) == 0) {
             const int64_t bk = orow * (K / 32) + col[b] / 32;
             ((float *)(out + L.d_off))[bk] = h2f(f2h(d[b]));

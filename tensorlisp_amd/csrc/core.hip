@@ -363,20 +363,20 @@ __global__ void __launch_bounds__(256) k_glu_quantize(const GluQuantArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) h[0][e] = 0.0f;
     }
-    const ActLayout L = act_layout(a.qo.type, nc, a.qo.rows, a.qo.f16);
+    const ActLayout L = act_layout(a.qo.type, nc, a.qo.rows);
     if (a.qo.type == TLH_TYPE_Q8_K) {  // nc % 256 == 0: every lane live
         uint32_t pk[1];
         int ps[1];
         float dd[1];
         q8K_waves<1>(h, lane, pk, ps, dd);
-        q8K_store_split((char *)a.qo.out, L, nc, row, ch, lane, pk[0], ps[0], dd[0], a.qo.f16);
+        q8K_store_split((char *)a.qo.out, L, nc, row, ch, lane, pk[0], ps[0], dd[0]);
     } else {
         const bool lv[1] = {live};
         const int64_t col[1] = {c0};
         if (a.qo.type == TLH_TYPE_Q8_1)
-            q80_quads_store_split<1, true>(h, lv, lane, (char *)a.qo.out, L, nc, row, col, a.qo.f16);
+            q80_quads_store_split<1, true>(h, lv, lane, (char *)a.qo.out, L, nc, row, col);
         else
-            q80_quads_store_split<1, false>(h, lv, lane, (char *)a.qo.out, L, nc, row, col, a.qo.f16);
+            q80_quads_store_split<1, false>(h, lv, lane, (char *)a.qo.out, L, nc, row, col);
     }
 }
 
@@ -1102,7 +1102,7 @@ __global__ void __launch_bounds__(256) k_norm_chain(const NormChainArgs a) {
         // the row (n <= 4096: all of it): a q8_K super-block in the quantize
         // launch's lane layout, or four 8-lane q8_0 / q8_1 blocks
         const int64_t row = blockIdx.x + (int64_t)gridDim.x * blockIdx.y;  // = the activation row
-        const ActLayout QL = act_layout(a.qo.type, n, a.qo.rows, a.qo.f16);
+        const ActLayout QL = act_layout(a.qo.type, n, a.qo.rows);
         const int lane = t & 63, w = t >> 6;
         if (a.qo.type == TLH_TYPE_Q8_K && split) {
 #pragma unroll
@@ -1114,7 +1114,7 @@ __global__ void __launch_bounds__(256) k_norm_chain(const NormChainArgs a) {
                 float d[1];
                 q8K_waves<1>(cj, lane, pk, ps, d);
                 if (1024 * j + 256 * w < n)  // wave-uniform (n % 256 == 0)
-                    q8K_store_split((char *)a.qo.out, QL, n, row, 4 * j + w, lane, pk[0], ps[0], d[0], a.qo.f16);
+                    q8K_store_split((char *)a.qo.out, QL, n, row, 4 * j + w, lane, pk[0], ps[0], d[0]);
             }
         } else if (a.qo.type == TLH_TYPE_Q8_K) {
             uint32_t pk[NC_CACHE];
@@ -1124,7 +1124,7 @@ __global__ void __launch_bounds__(256) k_norm_chain(const NormChainArgs a) {
 #pragma unroll
             for (int j = 0; j < NC_CACHE; ++j)
                 if (1024 * j + 256 * w < n)  // wave-uniform (n % 256 == 0)
-                    q8K_store_split((char *)a.qo.out, QL, n, row, 4 * j + w, lane, pk[j], ps[j], d[j], a.qo.f16);
+                    q8K_store_split((char *)a.qo.out, QL, n, row, 4 * j + w, lane, pk[j], ps[j], d[j]);
         } else {
             bool live[NC_CACHE];
             int64_t col[NC_CACHE];
@@ -1134,9 +1134,9 @@ __global__ void __launch_bounds__(256) k_norm_chain(const NormChainArgs a) {
                 live[j] = col[j] < n && mine(j);  // whole 8-lane groups (n % 32 == 0)
             }
             if (a.qo.type == TLH_TYPE_Q8_1)
-                q80_quads_store_split<NC_CACHE, true>(c, live, lane, (char *)a.qo.out, QL, n, row, col, a.qo.f16);
+                q80_quads_store_split<NC_CACHE, true>(c, live, lane, (char *)a.qo.out, QL, n, row, col);
             else
-                q80_quads_store_split<NC_CACHE, false>(c, live, lane, (char *)a.qo.out, QL, n, row, col, a.qo.f16);
+                q80_quads_store_split<NC_CACHE, false>(c, live, lane, (char *)a.qo.out, QL, n, row, col);
         }
     }
     for (int i = 4 * 256 * NC_CACHE + 4 * t; i < n; i += 4 * 256)

@@ -69,8 +69,8 @@ struct Dispatch {
     tlh_op nop, gop;
     Place nsrc[4], ndst, gdst;
     // D_CORE GLU, D_NORM_CHAIN: also quantizes its output for a MUL_MAT (type,
-    // activation rows, f16 codes) into that MUL_MAT's scratch block
-    int nq_type = 0, nq_f16 = 0;
+    // activation rows) into that MUL_MAT's scratch block
+    int nq_type = 0;
     int64_t nq_rows = 0;
     int64_t rt_off = 0;  // batched epilogue: byte offset of its rotation table in the program's table buffer
     tlh_op nq_op;          // that MUL_MAT (its quantize launch, if the fused form is refused)
@@ -1003,13 +1003,10 @@ class Lowering {
             bool many = false;  // a prefill's merged GEMM: its reduce stores (second paged stores allowed)
             if (batched) {
                 // 3..16 columns: the few-column kernel's stores; more (a
-                // prefill): the reduce of a q4_K / q5_K GEMM that splits K
-                int64_t rows = 0;
-                for (int k = 0; k < f.nmem; ++k) rows += f.mop[k].t[0].ne[1];
+                // prefill): the reduce of a q4_K / q5_K GEMM
                 const bool few = b.ne[1] >= 3 && b.ne[1] <= 16 &&
                                  (wty == TLH_TYPE_Q4_K || wty == TLH_TYPE_Q5_K || wty == TLH_TYPE_Q6_K);
-                many = b.ne[1] > 16 && (wty == TLH_TYPE_Q4_K || wty == TLH_TYPE_Q5_K) &&
-                       gemm_ksplit(wty, rows, b.ne[1], b.ne[0], 1) > 1;
+                many = b.ne[1] > 16 && (wty == TLH_TYPE_Q4_K || wty == TLH_TYPE_Q5_K);
                 if (!few && !many) continue;
             }
             const int64_t T = batched ? b.ne[1] : 1;  // tokens = columns
@@ -1225,6 +1222,14 @@ class Lowering {
             if (!batched) g.kind = D_GEMV_PRO;
             g.has_epi = 1;
             g.epi = e;
+            if (many) {  // its reduce reads the partials also of a GEMM that does not split K
+                const tlh_op *mops[3] = {&g.mop[0], &g.mop[1], &g.mop[2]};
+                g.scratch_bytes = std::max(g.scratch_bytes, mul_mat_compute_multi_scratch_bytes(mops, g.nmem, true));
+                if (g.block <= -2) {
+                    Group &gr = groups_[-2 - g.block];
+                    gr.bytes = std::max(gr.bytes, g.scratch_bytes);
+                }
+            }
             for (int k = 0; k < 3; ++k) g.edst[k] = edst[k], g.eidx[k] = eidx[k], g.edst2[k] = edst2[k];
             g.epos = epos;
             g.eff = eff;
@@ -1467,7 +1472,7 @@ class Lowering {
             if (pa) {
                 const int64_t per = (int64_t)g.pa.num_heads * g.pa.head_size;
                 if (g.block != -1 || K != per || rows != g.pa.num_seqs || !contiguous_f32(b) ||
-                    act_has_f16(wt, b.ne[1]) || !paged_attention_quantize_ok(g.pa, at))
+                    !paged_attention_quantize_ok(g.pa, at))
                     continue;
             } else {
                 const tlh_tensor &y = g.op.t[4];
@@ -1492,7 +1497,6 @@ class Lowering {
             }
             g.nq_type = at;
             g.nq_rows = rows;
-            g.nq_f16 = act_has_f16(wt, b.ne[1]);
             g.nq_op = q.op;
             g.block = q.block;
             Group &gr = groups_[-2 - q.block];
@@ -1827,7 +1831,6 @@ struct tlh_program {
                     qo.out = scratch;
                     qo.type = x.nq_type;
                     qo.rows = x.nq_rows;
-                    qo.f16 = x.nq_f16 != 0;
                 }
                 NormPartials qp;
                 if (x.pp_disp >= 0) {
@@ -1855,7 +1858,6 @@ struct tlh_program {
                     qo.out = scratch;
                     qo.type = x.nq_type;
                     qo.rows = x.nq_rows;
-                    qo.f16 = x.nq_f16 != 0;
                     char *own = (char *)scratch + x.pa_own;
                     st = launch_paged_attention(a, own, x.scratch_bytes - x.pa_own, s, (float *)dst, counters, &qo);
                     if (st == TLH_UNSUPPORTED) {
@@ -1999,7 +2001,6 @@ struct tlh_program {
                     qo.out = scratch;
                     qo.type = x.nq_type;
                     qo.rows = x.nq_rows;
-                    qo.f16 = x.nq_f16 != 0;
                     st = launch_glu_quantize(x.op, src[0], src[1], dst, qo, s);
                 } else {
                     st = tlh_core(x.core_kind, &x.op, src[0], src[1], src[2], dst, s);

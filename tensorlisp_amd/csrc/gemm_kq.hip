@@ -491,7 +491,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
     // row m of column n goes to obase + n * ostride + 4 m
     char *obase = (char *)a.dst + sl.i12 * a.d_nb2 + sl.i13 * a.d_nb3 + a.n0 * a.d_nb1;
     int64_t ostride = a.d_nb1;
-    if (nkc > 1) {
+    if (nkc > 1 || a.keep_part) {
         obase = (char *)(a.part + (kc * batches + batch) * a.N * a.M);
         ostride = 4 * a.M;
     } else if (a.nseg > 0) {
@@ -525,7 +525,7 @@ template <int WT> static tlh_status launch_kq(const MatmulArgs &a, int ks, hipSt
     case 64: launch_kq_tile<WT, 64, 64, 2, 2, 1, 2>(a, ks, stream); break;
     default: launch_kq_tile<WT, 128, 128, 4, 2, 1, 2>(a, ks, stream); break;
     }
-    return check_launch("gemm_kq");
+    return check_launch(WT == TLH_TYPE_Q4_K || WT == TLH_TYPE_Q5_K ? "gemm_q4k" : "gemm_kq");
 }
 
 // Tile shapes by columns. Up to 64 columns the weights' bytes set the time:
@@ -544,6 +544,8 @@ tlh_status launch_gemm_kq(const MatmulArgs &a, int ks, hipStream_t stream) {
     switch (a.wtype) {
     case TLH_TYPE_Q2_K: return launch_kq<TLH_TYPE_Q2_K>(a, ks, stream);
     case TLH_TYPE_Q3_K: return launch_kq<TLH_TYPE_Q3_K>(a, ks, stream);
+    case TLH_TYPE_Q4_K: return launch_kq<TLH_TYPE_Q4_K>(a, ks, stream);
+    case TLH_TYPE_Q5_K: return launch_kq<TLH_TYPE_Q5_K>(a, ks, stream);
     case TLH_TYPE_Q6_K: return launch_kq<TLH_TYPE_Q6_K>(a, ks, stream);
     default: return set_error(TLH_UNSUPPORTED, "gemm_kq: weight type %d", a.wtype);
     }

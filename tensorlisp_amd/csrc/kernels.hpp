@@ -34,9 +34,8 @@ int blocks_per_cu(Kern kern, int threads, size_t lds, std::atomic<int> &cache) {
 
 // rows of x (stride x_row_bytes) -> activation rows row_off.. of an output of
 // total_rows rows, in ggml's block layout or the split scratch layout.
-// f16: also write the codes as f16 (the scratch of a GEMM launch).
 tlh_status launch_quantize_act(int wtype, const float *x, int64_t K, int64_t rows, int64_t x_row_bytes, void *out,
-                               bool ggml_layout, int64_t row_off, int64_t total_rows, bool f16, hipStream_t stream);
+                               bool ggml_layout, int64_t row_off, int64_t total_rows, hipStream_t stream);
 tlh_status launch_dequantize(int type, const void *w, int64_t K, int64_t rows, int64_t w_row_bytes, float *y,
                              hipStream_t stream);
 
@@ -77,7 +76,8 @@ struct MatmulArgs {
     const char *ids;
     int64_t ids_nb0, ids_nb1, id_b1, id_nas;
     // K-split launches leave their partials in `part` without the chunk-sum
-    // launch (a consumer adds them: mul_mat_compute_keep)
+    // launch (a consumer adds them: mul_mat_compute_keep); the k-quant GEMM does
+    // so with one chunk too
     int keep_part;
 };
 
@@ -221,8 +221,8 @@ KqTile gemm_kq_tile(int64_t N);
 int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches);
 int64_t gemm_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches);
 tlh_status launch_gemm(const MatmulArgs &a, hipStream_t stream);  // any N, from the scratch
-// q4_K / q5_K GEMM whose K chunks' reduce stores through ep (the launch must
-// split K); TLH_UNSUPPORTED otherwise, before anything is launched
+// k-quant GEMM that leaves its K chunks (one or more) in a.part and whose
+// reduce stores through ep; TLH_UNSUPPORTED otherwise, before anything is launched
 tlh_status launch_gemm_epi(const MatmulArgs &a, const GemvEpi &ep, hipStream_t stream);
 
 // Dense FLASH_ATTN_EXT over f16 K/V (flash_attn.hip). Strides in bytes;
@@ -248,7 +248,8 @@ tlh_status launch_flash_attn(const FlashAttnDesc &d, hipStream_t stream);
 // type and K as one register-GEMV launch (tlhip.cpp); TLH_UNSUPPORTED when the
 // pointers do not allow it.
 bool mul_mat_compute_multi_ok(const tlh_op *const *ops, int n);
-size_t mul_mat_compute_multi_scratch_bytes(const tlh_op *const *ops, int n);
+// epi: with the partials the store epilogue's reduce reads, also of one chunk
+size_t mul_mat_compute_multi_scratch_bytes(const tlh_op *const *ops, int n, bool epi = false);
 tlh_status mul_mat_compute_multi(const tlh_op *const *ops, const void *const *w, void *const *dst, int n,
                                  const void *scratch, size_t scratch_bytes, hipStream_t stream,
                                  const GemvEpi *epi = nullptr);
@@ -277,13 +278,11 @@ tlh_status mul_mat_multi_pro(const tlh_op *const *ops, const void *const *w, voi
                              const GemvPro &pro, const void *x, hipStream_t stream);
 // A kernel's rows quantized as it writes them: the activation scratch of a
 // MUL_MAT (split layout of `type` = q8_0 / q8_1 / q8_K for `rows` activation
-// rows, f16 codes too when `f16`), row r of the kernel's output being
-// activation row r.
+// rows), row r of the kernel's output being activation row r.
 struct ActQuantOut {
     void *out = nullptr;
     int type = 0;
     int64_t rows = 0;
-    bool f16 = false;
 };
 // Longest row the norm chain quantizes (the row is held in registers).
 constexpr int64_t NORM_CHAIN_QUANT_MAX = 4096;

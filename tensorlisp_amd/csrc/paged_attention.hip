@@ -108,7 +108,7 @@ template <int HS, int W>
 __device__ __forceinline__ void quantize_heads(const float *sq, int gc, int num_heads, int head0, int seq, void *qout,
                                                int64_t qrows) {
     const int64_t K = (int64_t)num_heads * HS;
-    const ActLayout QL = act_layout(TLH_TYPE_Q8_K, K, qrows, false);
+    const ActLayout QL = act_layout(TLH_TYPE_Q8_K, K, qrows);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int b = wave; b < gc * HS / QKK; b += W) {
         float v[1][4];
@@ -118,8 +118,7 @@ __device__ __forceinline__ void quantize_heads(const float *sq, int gc, int num_
         int psum[1];
         float dq[1];
         q8K_waves<1>(v, lane, packed, psum, dq);
-        q8K_store_split((char *)qout, QL, K, seq, (int64_t)head0 * HS / QKK + b, lane, packed[0], psum[0], dq[0],
-                        false);
+        q8K_store_split((char *)qout, QL, K, seq, (int64_t)head0 * HS / QKK + b, lane, packed[0], psum[0], dq[0]);
     }
 }
 
@@ -522,7 +521,7 @@ size_t paged_attention_counters(const tlh_paged_attention_args &a) {
 tlh_status launch_paged_attention(const tlh_paged_attention_args &a, void *scratch, size_t, hipStream_t stream,
                                   float *out32, unsigned *counters, const ActQuantOut *qo) {
     float *s = (float *)scratch;
-    if (qo && (!counters || !qo->out || !paged_attention_quantize_ok(a, qo->type) || qo->f16 ||
+    if (qo && (!counters || !qo->out || !paged_attention_quantize_ok(a, qo->type) ||
                qo->rows < a.num_seqs))
         return set_error(TLH_UNSUPPORTED, "paged_attention: the merge quantizes whole q8_K blocks of heads, "
                                           "one launch, no f16 codes");

@@ -26,7 +26,7 @@ namespace tlh {
 template <bool GGML_LAYOUT, bool Q81>
 __global__ void __launch_bounds__(256) k_quantize_q8_0(const float *__restrict__ x, int64_t K, int64_t rows,
                                                        int64_t x_row_bytes, void *__restrict__ out, int64_t row_off,
-                                                       int64_t total_rows, bool f16) {
+                                                       int64_t total_rows) {
 #pragma clang fp contract(off)
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t total = K * rows;
@@ -57,10 +57,9 @@ __global__ void __launch_bounds__(256) k_quantize_q8_0(const float *__restrict__
             if (Q81) *(uint16_t *)(b + 2) = sh;
         }
     } else {
-        const ActLayout L = act_layout(Q81 ? TLH_TYPE_Q8_1 : TLH_TYPE_Q8_0, K, total_rows, f16);
+        const ActLayout L = act_layout(Q81 ? TLH_TYPE_Q8_1 : TLH_TYPE_Q8_0, K, total_rows);
         int8_t *qs = (int8_t *)out + L.qs_off;
         qs[orow * K + col] = (int8_t)q;
-        if (f16) ((_Float16 *)((char *)out + L.q16_off))[orow * K + col] = (_Float16)q;
         if (lane32 == 0) {
             ((float *)((char *)out + L.d_off))[orow * (K / QK) + blk] = h2f(dh);
             ((int32_t *)((char *)out + L.sum_off))[orow * (K / QK) + blk] = Q81 ? __float_as_int(h2f(sh)) : s;
@@ -76,7 +75,7 @@ __global__ void __launch_bounds__(256) k_quantize_q8_0(const float *__restrict__
 template <bool GGML_LAYOUT>
 __global__ void __launch_bounds__(256) k_quantize_q8_K(const float *__restrict__ x, int64_t K, int64_t rows,
                                                        int64_t x_row_bytes, void *__restrict__ out, int64_t row_off,
-                                                       int64_t total_rows, bool f16) {
+                                                       int64_t total_rows) {
 #pragma clang fp contract(off)
     const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int lane = threadIdx.x & 63;
@@ -99,8 +98,8 @@ __global__ void __launch_bounds__(256) k_quantize_q8_K(const float *__restrict__
         if ((lane & 3) == 0) *(int16_t *)(b + 4 + QKK + 2 * (lane >> 2)) = (int16_t)psum[0];
         if (lane == 0) *(float *)b = d[0];
     } else {
-        q8K_store_split((char *)out, act_layout(TLH_TYPE_Q8_K, K, total_rows, f16), K, orow, blk, lane, packed[0],
-                        psum[0], d[0], f16);
+        q8K_store_split((char *)out, act_layout(TLH_TYPE_Q8_K, K, total_rows), K, orow, blk, lane, packed[0],
+                        psum[0], d[0]);
     }
 }
 
@@ -125,22 +124,22 @@ static inline unsigned grid_for(int64_t threads, int per_block) {
 }
 
 tlh_status launch_quantize_act(int wtype, const float *x, int64_t K, int64_t rows, int64_t x_row_bytes, void *out,
-                               bool ggml_layout, int64_t row_off, int64_t total_rows, bool f16, hipStream_t stream) {
+                               bool ggml_layout, int64_t row_off, int64_t total_rows, hipStream_t stream) {
     if (rows == 0 || K == 0) return TLH_OK;
     if (vec_dot_type(wtype) == TLH_TYPE_Q8_0 || vec_dot_type(wtype) == TLH_TYPE_Q8_1) {
         const unsigned g = grid_for(K * rows, 256);
         const bool q81 = vec_dot_type(wtype) == TLH_TYPE_Q8_1;
         auto kern = ggml_layout ? (q81 ? k_quantize_q8_0<true, true> : k_quantize_q8_0<true, false>)
                                 : (q81 ? k_quantize_q8_0<false, true> : k_quantize_q8_0<false, false>);
-        hipLaunchKernelGGL(kern, dim3(g), dim3(256), 0, stream, x, K, rows, x_row_bytes, out, row_off, total_rows, f16);
+        hipLaunchKernelGGL(kern, dim3(g), dim3(256), 0, stream, x, K, rows, x_row_bytes, out, row_off, total_rows);
     } else {
         const unsigned g = grid_for((K / QKK) * rows * 64, 256);
         if (ggml_layout)
             hipLaunchKernelGGL(k_quantize_q8_K<true>, dim3(g), dim3(256), 0, stream, x, K, rows, x_row_bytes, out,
-                               row_off, total_rows, f16);
+                               row_off, total_rows);
         else
             hipLaunchKernelGGL(k_quantize_q8_K<false>, dim3(g), dim3(256), 0, stream, x, K, rows, x_row_bytes, out,
-                               row_off, total_rows, f16);
+                               row_off, total_rows);
     }
     return check_launch("quantize_act");
 }

@@ -443,7 +443,11 @@ tlh_status tlh_stream_sync(void *stream) {
 static int64_t mm_float_row(const MulMatShape &s) { return align_up(s.K * float_size(s.wtype), 16); }
 static int64_t mm_act_bytes(const MulMatShape &s) {
     if (s.flt) return align_up(s.act_rows * mm_float_row(s), 256);
-    return act_layout(s.act_type, s.K, s.act_rows, act_has_f16(s.wtype, s.N)).total;
+    // q4_K / q5_K above 16 columns: with room for the codes and bsums in f16 as
+    // well, which the sizes told to callers (and so what tlh_mul_mat_noalloc
+    // refuses) have always included
+    const bool f16 = s.N > 16 && (s.wtype == TLH_TYPE_Q4_K || s.wtype == TLH_TYPE_Q5_K);
+    return act_layout(s.act_type, s.K, s.act_rows).total + (f16 ? align_up(s.act_rows * (s.K + s.K / 16) * 2, 256) : 0);
 }
 static FloatMM float_mm(const tlh_op *op, const MulMatShape &s, const void *src0, const void *x, int xtype,
                         const int64_t (&x_nb)[4], void *dst) {
@@ -497,12 +501,12 @@ static tlh_status mm_quantize(const tlh_op *op, const MulMatShape &s, const void
     const bool packed = b.nb[2] == b.nb[1] * s.N && b.nb[3] == b.nb[2] * s.ne12;
     if (packed)
         return launch_quantize_act(a.ty, (const float *)src1, s.K, s.act_rows, b.nb[1], scratch, false, 0,
-                                   s.act_rows, act_has_f16(s.wtype, s.N), hs);
+                                   s.act_rows, hs);
     for (int64_t i13 = 0; i13 < s.ne13; ++i13)
         for (int64_t i12 = 0; i12 < s.ne12; ++i12) {
             const float *x = (const float *)((const char *)src1 + i12 * b.nb[2] + i13 * b.nb[3]);
             const tlh_status st = launch_quantize_act(a.ty, x, s.K, s.N, b.nb[1], scratch, false,
-                                                      s.N * (i12 + s.ne12 * i13), s.act_rows, act_has_f16(s.wtype, s.N), hs);
+                                                      s.N * (i12 + s.ne12 * i13), s.act_rows, hs);
             if (st != TLH_OK) return st;
         }
     return TLH_OK;
@@ -569,8 +573,8 @@ bool tlh::mul_mat_compute_multi_ok(const tlh_op *const *ops, int n) {
         MulMatShape s;
         if (check_mul_mat(ops[i], s) != TLH_OK || mm_empty(s) || s.flt || s.N < 3 || s.ne12 * s.ne13 != 1)
             return false;
-        // more than 16 columns: the q4_K / q5_K GEMM over the segments' rows
-        // (each but the last a whole number of its 128-row tiles)
+        // more than 16 columns: the k-quant GEMM over the segments' rows (each
+        // but the last a whole number of its 128-row tiles), q4_K / q5_K
         const bool gemm = s.N > 16;
         if (gemm ? !(s.wtype == TLH_TYPE_Q4_K || s.wtype == TLH_TYPE_Q5_K)
                  : gemv_mfma_partial_bytes(s.K, s.M, s.N, 1) != 0)
@@ -586,20 +590,21 @@ bool tlh::mul_mat_compute_multi_ok(const tlh_op *const *ops, int n) {
 
 // The quantized activation of the first node plus, for the GEMM form, the
 // partial sums of its K chunks over all the nodes' rows.
-size_t tlh::mul_mat_compute_multi_scratch_bytes(const tlh_op *const *ops, int n) {
+size_t tlh::mul_mat_compute_multi_scratch_bytes(const tlh_op *const *ops, int n, bool epi) {
     if (!mul_mat_compute_multi_ok(ops, n)) return 0;
     MulMatShape s;
     check_mul_mat(ops[0], s);
     int64_t rows = 0;
     for (int i = 0; i < n; ++i) rows += ops[i]->t[0].ne[1];
-    const int64_t part = s.N > 16 ? align_up(gemm_partial_bytes(s.wtype, rows, s.N, s.K, 1), 256) : 0;
+    int64_t part = s.N > 16 ? gemm_partial_bytes(s.wtype, rows, s.N, s.K, 1) : 0;
+    if (s.N > 16 && epi && part == 0) part = s.N * rows * 4;
+    part = align_up(part, 256);
     return (size_t)(mm_act_bytes(s) + part);
 }
 
 // With epi (the executor's batched Q / K / V projection): the few-column
 // kernel stores through the epilogue (N <= 16, one K chunk), or above 16
-// columns the q4_K / q5_K GEMM's K-chunk reduce does (the GEMM must split K);
-// TLH_UNSUPPORTED when neither can take the shapes or pointers (the executor
+// columns the k-quant GEMM's reduce does; TLH_UNSUPPORTED when neither can take the shapes or pointers (the executor
 // then runs the absorbed dispatches after a plain launch).
 tlh_status tlh::mul_mat_compute_multi(const tlh_op *const *ops, const void *const *w, void *const *dst, int n,
                                       const void *scratch, size_t scratch_bytes, hipStream_t stream,
@@ -616,7 +621,7 @@ tlh_status tlh::mul_mat_compute_multi(const tlh_op *const *ops, const void *cons
     }
     MulMatShape s;
     check_mul_mat(ops[0], s);
-    const size_t need = mul_mat_compute_multi_scratch_bytes(ops, n);
+    const size_t need = mul_mat_compute_multi_scratch_bytes(ops, n, epi != nullptr);
     if (!scratch || scratch_bytes < need)
         return set_error(TLH_INVALID, "mul_mat_compute_multi: scratch of %zu bytes, need %zu", scratch_bytes, need);
     if ((uintptr_t)scratch & 255) return set_error(TLH_INVALID, "mul_mat_compute_multi: scratch must be 256-byte aligned");
@@ -987,11 +992,11 @@ tlh_status tlh_mul_mat_id(const tlh_op *op, const void *src0, const void *src1, 
     const hipStream_t hs = (hipStream_t)stream;
     const int64_t rows = s.n_b1 * s.n_tok;
     if (b.nb[2] == b.nb[1] * s.n_b1 || s.n_tok == 1) {
-        st = launch_quantize_act(a.ty, (const float *)src1, s.K, rows, b.nb[1], scratch, false, 0, rows, false, hs);
+        st = launch_quantize_act(a.ty, (const float *)src1, s.K, rows, b.nb[1], scratch, false, 0, rows, hs);
     } else {
         for (int64_t t = 0; t < s.n_tok && st == TLH_OK; ++t)
             st = launch_quantize_act(a.ty, (const float *)((const char *)src1 + t * b.nb[2]), s.K, s.n_b1, b.nb[1],
-                                     scratch, false, s.n_b1 * t, rows, false, hs);
+                                     scratch, false, s.n_b1 * t, rows, hs);
     }
     if (st != TLH_OK) return st;
     MatmulArgs m{};
@@ -1030,7 +1035,7 @@ tlh_status tlh_quantize_act(int wtype, const float *x, int64_t k, int64_t rows, 
     if ((!x || !y) && k * rows > 0) return set_error(TLH_INVALID, "quantize_act: null pointer");
     if (x_row_bytes < 4 * k || (x_row_bytes & 3) || ((uintptr_t)x & 3) || ((uintptr_t)y & 3))
         return set_error(TLH_INVALID, "quantize_act: rows must be 4-byte aligned f32 with stride >= 4k");
-    return launch_quantize_act(wtype, x, k, rows, x_row_bytes, y, true, 0, rows, false, (hipStream_t)stream);
+    return launch_quantize_act(wtype, x, k, rows, x_row_bytes, y, true, 0, rows, (hipStream_t)stream);
 }
 
 tlh_status tlh_dequantize(int type, const void *w, int64_t k, int64_t rows, int64_t w_row_bytes, float *y,

@@ -13,12 +13,12 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from refs import NAMES, Q2_K, Q3_K, Q6_K, oracle
+from refs import NAMES, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, oracle
 from tensorlisp_amd import native as N
 from tensorlisp_amd import synth
 
 pytestmark = pytest.mark.gpu
-TYPES = (Q2_K, Q3_K, Q6_K)
+TYPES = (Q2_K, Q3_K, Q4_K, Q5_K, Q6_K)
 
 
 def dev(a):
@@ -30,7 +30,7 @@ def dev(a):
 def bound(t, w, K, x):
     o = oracle()
     wd = np.abs(o.dequantize(t, w, K)).astype(np.float64)
-    if t == Q2_K:  # scale and min terms are added apart: their sizes, not their difference's
+    if t in (Q2_K, Q4_K, Q5_K):  # scale and min terms are added apart: their sizes, not their difference's
         wd = wd + 2 * np.abs(wd).max()
     return 2 * (K // 256 + 8) * 2.0 ** -23 * (np.abs(x).astype(np.float64) @ wd.T) * (128 / 127)
 
@@ -64,9 +64,9 @@ def test_extreme_codes(gpu, t, n):
     -128 * -32 are the largest scaled codes) against activation codes of +-127."""
     M, K = 70, 512
     w = synth.random_blocks(t, 5, M, K).reshape(-1, N.BLOCK[t][1]).copy()
-    sc = {Q2_K: slice(0, 16), Q3_K: slice(96, 108), Q6_K: slice(192, 208)}[t]
-    fill = {Q2_K: (0xFF, 0x0F), Q3_K: (0x00, 0xFF), Q6_K: (0x80, 0x7F)}[t]
-    d = {Q2_K: slice(80, 84), Q3_K: slice(108, 110), Q6_K: slice(208, 210)}[t]
+    sc = {Q2_K: slice(0, 16), Q3_K: slice(96, 108), Q4_K: slice(4, 16), Q5_K: slice(4, 16), Q6_K: slice(192, 208)}[t]
+    fill = {Q2_K: (0xFF, 0x0F), Q3_K: (0x00, 0xFF), Q4_K: (0xFF, 0x3F), Q5_K: (0xFF, 0x3F), Q6_K: (0x80, 0x7F)}[t]
+    d = {Q2_K: slice(80, 84), Q3_K: slice(108, 110), Q4_K: slice(0, 4), Q5_K: slice(0, 4), Q6_K: slice(208, 210)}[t]
     keep = w[:, d].copy()
     for i in range(w.shape[0]):
         w[i] = 0x00 if i % 3 == 0 else 0xFF if i % 3 == 1 else w[i]
