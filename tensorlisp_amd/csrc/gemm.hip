@@ -36,7 +36,7 @@ tlh_status launch_gemm_epi(const MatmulArgs &a, const GemvEpi &ep, hipStream_t s
     if (st != TLH_OK) return st;
     MatmulArgs g = a;
     g.keep_part = 1;  // one chunk's sums go through the reduce's stores too
-    st = launch_gemm_kq(g, ks, stream);
+    st = launch_gemm_kq(g, gemm_kq_tile(a.N).bn, ks, stream);
     return st != TLH_OK ? st : launch_partial_reduce_epi(a, ks, ep, stream);
 }
 
@@ -45,7 +45,7 @@ tlh_status launch_gemm(const MatmulArgs &a, hipStream_t stream) {
     if (has_gemm(a.wtype)) {
         const int ks = gemm_ksplit(a.wtype, a.M, a.N, a.K, batches);
         if (ks > 1 && !a.part) return set_error(TLH_INVALID, "gemm: a K split of %d needs a partials buffer", ks);
-        const tlh_status st = kquant_type(a.wtype) ? launch_gemm_kq(a, ks, stream) : launch_gemm_q8(a, ks, stream);
+        const tlh_status st = kquant_type(a.wtype) ? launch_gemm_kq(a, gemm_kq_tile(a.N).bn, ks, stream) : launch_gemm_q8(a, ks, stream);
         return st != TLH_OK || ks == 1 || a.keep_part ? st : launch_partial_reduce(a, ks, stream);
     }
     if (a.keep_part) return set_error(TLH_UNSUPPORTED, "gemm: no kept partials for weight type %d", a.wtype);
@@ -57,6 +57,63 @@ tlh_status launch_gemm(const MatmulArgs &a, hipStream_t stream) {
         if (st != TLH_OK) return st;
     }
     return TLH_OK;
+}
+
+// MUL_MAT_ID's (expert, token) pairs by expert: one workgroup counts the pairs
+// of each expert, gives every expert its run of the pair list and its column
+// tiles (bn pairs each), and deals the pairs out. The order of an expert's
+// pairs is not fixed; each pair's outputs depend on its own column only.
+constexpr int GP_THREADS = 1024;
+__global__ void __launch_bounds__(GP_THREADS) k_group_plan(const MatmulArgs a, int bn, int32_t *plan) {
+    __shared__ int cnt[GROUP_MAX_EXPERTS + 1], first[GROUP_MAX_EXPERTS + 1];
+    __shared__ int wave_pairs[16], wave_tiles[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n_as = (int)a.id_nas, used = (int)a.ne12, pairs = used * (int)a.ne13;
+    auto expert = [&](int p) {
+        const int t = p / used, e = *(const int32_t *)(a.ids + (int64_t)(p - t * used) * a.ids_nb0 + (int64_t)t * a.ids_nb1);
+        return (unsigned)e < (unsigned)n_as ? e : n_as;
+    };
+    for (int i = tid; i <= n_as; i += GP_THREADS) cnt[i] = 0;
+    __syncthreads();
+    for (int p = tid; p < pairs; p += GP_THREADS) atomicAdd(&cnt[expert(p)], 1);
+    __syncthreads();
+    int32_t *tile = plan + 4, *list = tile + 4 * a.grp_tiles;
+    int done_pairs = 0, done_tiles = 0;
+    for (int e0 = 0; e0 <= n_as; e0 += GP_THREADS) {  // exclusive sums of pairs and tiles over the experts
+        const int e = e0 + tid, c = e <= n_as ? cnt[e] : 0, nt = (c + bn - 1) / bn;
+        int sp = c, st = nt;
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+            const int up = __shfl_up(sp, m, 64), ut = __shfl_up(st, m, 64);
+            if (lane >= m) sp += up, st += ut;
+        }
+        if (lane == 63) wave_pairs[wave] = sp, wave_tiles[wave] = st;
+        __syncthreads();
+        int bp = done_pairs, bt = done_tiles;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) bp += wave_pairs[w], bt += wave_tiles[w];
+            done_pairs += wave_pairs[w], done_tiles += wave_tiles[w];
+        }
+        if (e <= n_as) {
+            first[e] = bp + sp - c;
+            for (int i = 0; i < nt; ++i) {
+                const int left = c - i * bn;
+                int32_t *t = tile + 4 * (int64_t)(bt + st - nt + i);
+                t[0] = e < n_as ? e : -1;
+                t[1] = bp + sp - c + i * bn;
+                t[2] = left < bn ? left : bn;
+                t[3] = 0;
+            }
+        }
+        __syncthreads();
+    }
+    if (tid == 0) plan[0] = done_tiles;
+    for (int p = tid; p < pairs; p += GP_THREADS) list[atomicAdd(&first[expert(p)], 1)] = p;
+}
+
+tlh_status launch_group_plan(const MatmulArgs &a, int64_t bn, int32_t *plan, hipStream_t stream) {
+    hipLaunchKernelGGL(k_group_plan, dim3(1), dim3(GP_THREADS), 0, stream, a, (int)bn, plan);
+    return check_launch("group_plan");
 }
 
 }  // namespace tlh

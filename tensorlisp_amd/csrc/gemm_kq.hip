@@ -9,12 +9,7 @@
 // The scaled code sc_s * q of an element is formed once per workgroup as it
 // is staged to LDS, as one or two int8 planes, so that the products of a whole
 // super-block run on v_mfma_i32_32x32x32_i8 without any per-sub-block scaling
-// between them, exact in int32:
-//   q2_K  sc * q <= 45: one plane
-//   q3_K  -(sc * (q - 4)) in -128..124: one plane (negated, so that it fits)
-//   q4_K  sc = 8 sh + sl: planes sh * q and sl * q (<= 105), S = 8 H + L;
-//         a plane of four nibbles is one packed 16-bit multiply (no byte carries)
-//   q5_K, q6_K  sc * q (13 bits): high and (signed) low byte, S = 256 H + L
+// between them, exact in int32 (the planes: kq_unit.hpp).
 // Mn is one f16 MFMA per super-block (A = bsums, |.| <= 2032, B = the mins;
 // exact). The f32 finalize runs once per super-block, as on the CPU.
 //
@@ -23,182 +18,9 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "kq_unit.hpp"
 
 namespace tlh {
-
-typedef int kq_v4i __attribute__((ext_vector_type(4)));
-typedef int kq_v16i __attribute__((ext_vector_type(16)));
-typedef float kq_v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 kq_v8h __attribute__((ext_vector_type(8)));
-typedef uint32_t kq_u4 __attribute__((ext_vector_type(4)));  // (plain vectors: a struct of them stays in registers)
-typedef uint32_t kq_u2 __attribute__((ext_vector_type(2)));
-typedef unsigned short kq_u16x2 __attribute__((ext_vector_type(2)));
-
-template <int WT> constexpr int kq_planes() { return WT == TLH_TYPE_Q2_K || WT == TLH_TYPE_Q3_K ? 1 : 2; }
-template <int WT> constexpr bool kq_has_min() { return WT == TLH_TYPE_Q2_K || WT == TLH_TYPE_Q4_K || WT == TLH_TYPE_Q5_K; }
-
-// A unit is 32 elements of a weight row's half super-block (128 elements): two
-// groups of 16 with one scale each. Unit u of half h reads 16 code bytes (and
-// 16 bytes of high bits) and fills 16-byte chunks G0 and G1 of the row's LDS
-// row of 128 codes.
-template <int WT> struct KqUnit {
-    kq_u4 q;
-    kq_u4 hi;       // q3_K hmask, q5_K qh, q6_K qh
-    uint32_t s[5];  // header words: scales, d / dmin
-};
-
-__device__ __forceinline__ kq_u4 kq_ld16(const void *p) {
-    kq_u4 v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
-}
-template <typename T> __device__ __forceinline__ T kq_ld(const void *p) {
-    T v;
-    __builtin_memcpy(&v, p, sizeof v);
-    return v;
-}
-
-template <int WT, int HALF> __device__ __forceinline__ void kq_fetch(const uint8_t *blk, int u, KqUnit<WT> &r) {
-    if constexpr (WT == TLH_TYPE_Q4_K || WT == TLH_TYPE_Q5_K) {
-        const kq_u4 h = kq_ld16(blk);
-        r.s[0] = h.x, r.s[1] = h.y, r.s[2] = h.z, r.s[3] = h.w;
-        r.q = kq_ld16(blk + (WT == TLH_TYPE_Q5_K ? 48 : 16) + 64 * HALF + 16 * u);
-        if constexpr (WT == TLH_TYPE_Q5_K) r.hi = kq_ld16(blk + 16 + 16 * (u & 1));
-    } else if constexpr (WT == TLH_TYPE_Q6_K) {
-        r.q = kq_ld16(blk + 64 * HALF + 16 * u);
-        r.hi = kq_ld16(blk + 128 + 32 * HALF + 16 * (u & 1));
-        const kq_u2 s = kq_ld<kq_u2>(blk + 192 + 8 * HALF);
-        r.s[0] = s.x, r.s[1] = s.y;
-        if constexpr (HALF == 1) r.s[2] = kq_ld<uint16_t>(blk + 208);
-    } else if constexpr (WT == TLH_TYPE_Q2_K) {
-        const kq_u4 s = kq_ld16(blk);
-        r.s[0] = s.x, r.s[1] = s.y, r.s[2] = s.z, r.s[3] = s.w;
-        r.q = kq_ld16(blk + 16 + 32 * HALF + 16 * (u & 1));
-        if constexpr (HALF == 1) r.s[4] = kq_ld<uint32_t>(blk + 80);
-    } else {  // q3_K
-        r.hi = kq_ld16(blk + 16 * (u & 1));
-        r.q = kq_ld16(blk + 32 + 32 * HALF + 16 * (u & 1));
-        r.s[0] = kq_ld<uint32_t>(blk + 96), r.s[1] = kq_ld<uint32_t>(blk + 100), r.s[2] = kq_ld<uint32_t>(blk + 104);
-        if constexpr (HALF == 1) r.s[3] = kq_ld<uint16_t>(blk + 108);
-    }
-}
-
-// The unit's first chunk (of 8 per LDS row); the second is kq_gap chunks on.
-template <int WT> __device__ __forceinline__ int kq_chunk(int u) {
-    return WT == TLH_TYPE_Q6_K ? u : 4 * (u >> 1) + (u & 1);
-}
-template <int WT> constexpr int kq_gap() { return WT == TLH_TYPE_Q6_K ? 4 : 2; }
-
-__device__ __forceinline__ uint32_t kq_mul2(uint32_t a, uint32_t b) {  // 16-bit lanes, modulo 2^16
-    return __builtin_bit_cast(uint32_t, (kq_u16x2)(__builtin_bit_cast(kq_u16x2, a) * __builtin_bit_cast(kq_u16x2, b)));
-}
-__device__ __forceinline__ uint32_t kq_mad2(uint32_t a, uint32_t b, uint32_t c) {
-    return __builtin_bit_cast(uint32_t, (kq_u16x2)(__builtin_bit_cast(kq_u16x2, a) * __builtin_bit_cast(kq_u16x2, b) +
-                                                    __builtin_bit_cast(kq_u16x2, c)));
-}
-__device__ __forceinline__ uint32_t kq_twice(int v) { return (uint32_t)(v & 0xffff) * 0x10001u; }
-
-// Four codes c (one a byte) times sc plus `off` in 16 bits each; the results'
-// high bytes to h, low bytes to l.
-__device__ __forceinline__ void kq_wide(uint32_t c, uint32_t sc2, uint32_t off2, uint32_t &h, uint32_t &l) {
-    const uint32_t a = __builtin_amdgcn_perm(0u, c, 0x0c010c00u), b = __builtin_amdgcn_perm(0u, c, 0x0c030c02u);
-    const uint32_t va = kq_mad2(a, sc2, off2), vb = kq_mad2(b, sc2, off2);
-    h = __builtin_amdgcn_perm(vb, va, 0x07050301u);
-    l = __builtin_amdgcn_perm(vb, va, 0x06040200u);
-}
-
-// The unit's scaled codes: out[plane][group][dword].
-template <int WT, int HALF>
-__device__ __forceinline__ void kq_codes(const KqUnit<WT> &r, int u, uint32_t (&out)[2][2][4]) {
-    const uint32_t q[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
-    const uint32_t hi[4] = {r.hi.x, r.hi.y, r.hi.z, r.hi.w};
-    if constexpr (WT == TLH_TYPE_Q4_K || WT == TLH_TYPE_Q5_K) {
-        // scales of the half's four sub-blocks, then of 2 (u >> 1) and the next
-        const uint32_t sc4 = HALF == 0 ? r.s[1] & 0x3f3f3f3fu : (r.s[3] & 0x0f0f0f0fu) | ((r.s[1] >> 2) & 0x30303030u);
-        const uint32_t two = sc4 >> (16 * (u >> 1));
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const uint32_t sc = (two >> (8 * g)) & 0xff;
-            if constexpr (WT == TLH_TYPE_Q4_K) {
-                const uint32_t sh2 = (sc >> 3) * 0x10001u, sl2 = (sc & 7) * 0x10001u;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t c = (g == 0 ? q[i] : q[i] >> 4) & 0x0f0f0f0fu;
-                    out[0][g][i] = kq_mul2(c, sh2);
-                    out[1][g][i] = kq_mul2(c, sl2);
-                }
-            } else {
-                // the low byte as a signed one: + 128 before, its sign bit flipped after
-                const uint32_t sc2 = sc * 0x10001u;
-                const int bit = 4 * HALF + 2 * (u >> 1) + g;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t c = ((g == 0 ? q[i] : q[i] >> 4) & 0x0f0f0f0fu) | (((hi[i] >> bit) & 0x01010101u) << 4);
-                    kq_wide(c, sc2, 0x00800080u, out[0][g][i], out[1][g][i]);
-                    out[1][g][i] ^= 0x80808080u;
-                }
-            }
-        }
-    } else if constexpr (WT == TLH_TYPE_Q6_K) {
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const int sc = (int)(int8_t)((g == 0 ? r.s[0] : r.s[1]) >> (8 * u));
-            const uint32_t sc2 = kq_twice(sc), off2 = kq_twice(128 - 32 * sc);
-            const int sh = 4 * g + 2 * (u >> 1);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t c = ((g == 0 ? q[i] : q[i] >> 4) & 0x0f0f0f0fu) | (((hi[i] >> sh) & 0x03030303u) << 4);
-                kq_wide(c, sc2, off2, out[0][g][i], out[1][g][i]);
-                out[1][g][i] ^= 0x80808080u;
-            }
-        }
-    } else if constexpr (WT == TLH_TYPE_Q2_K) {
-        const uint32_t sc4 = ((u >> 1) ? r.s[2 * HALF + 1] : r.s[2 * HALF]) & 0x0f0f0f0fu;
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const uint32_t sc2 = ((sc4 >> (8 * ((u & 1) + 2 * g))) & 0xff) * 0x10001u;
-            const int sh = 2 * (2 * (u >> 1) + g);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) out[0][g][i] = kq_mul2((q[i] >> sh) & 0x03030303u, sc2);
-        }
-    } else {  // q3_K
-        const uint32_t lo = (u >> 1) ? r.s[1] : r.s[0];
-        const uint32_t sc4 = ((HALF ? lo >> 4 : lo) & 0x0f0f0f0fu) | (((r.s[2] >> (4 * HALF + 2 * (u >> 1))) & 0x03030303u) << 4);
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const int sc = (int)((sc4 >> (8 * ((u & 1) + 2 * g))) & 0xff) - 32;
-            const uint32_t sc2 = kq_twice(-sc), off2 = kq_twice(4 * sc);
-            const int j = 2 * (u >> 1) + g;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t c = ((q[i] >> (2 * j)) & 0x03030303u) | (((hi[i] >> (4 * HALF + j)) & 0x01010101u) << 2);
-                uint32_t h;
-                kq_wide(c, sc2, off2, h, out[0][g][i]);
-            }
-        }
-    }
-}
-
-// A row's d, dmin and the 16 mins of its bsums (q4 / q5_K: each of 8 mins
-// twice), from the second half's header.
-template <int WT> __device__ __forceinline__ void kq_row_meta(const KqUnit<WT> &r, float &d, float &dmin, uint32_t (&mn)[4]) {
-    dmin = 0.0f;
-    if constexpr (WT == TLH_TYPE_Q4_K || WT == TLH_TYPE_Q5_K) {
-        d = h2f((uint16_t)(r.s[0] & 0xffff));
-        dmin = h2f((uint16_t)(r.s[0] >> 16));
-        mn[0] = r.s[2] & 0x3f3f3f3fu;
-        mn[1] = ((r.s[3] >> 4) & 0x0f0f0f0fu) | ((r.s[2] >> 2) & 0x30303030u);
-    } else if constexpr (WT == TLH_TYPE_Q6_K) {
-        d = h2f((uint16_t)r.s[2]);
-    } else if constexpr (WT == TLH_TYPE_Q2_K) {
-        d = h2f((uint16_t)(r.s[4] & 0xffff));
-        dmin = h2f((uint16_t)(r.s[4] >> 16));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) mn[i] = (r.s[i] >> 4) & 0x0f0f0f0fu;
-    } else {
-        d = h2f((uint16_t)r.s[3]);
-    }
-}
 
 // Tile of BM weight rows x BN tokens per workgroup of WM x WN x WK waves: a
 // wave owns BM / WM rows and BN / WN tokens in 32 x 32 MFMA tiles, and of each
@@ -210,7 +32,9 @@ template <int WT> __device__ __forceinline__ void kq_row_meta(const KqUnit<WT> &
 // LDS-only barrier a stage. LDS rows are 128 bytes, chunk c of row r at
 // position c ^ (r & 7), so that 8 consecutive rows' operand reads hit
 // distinct banks.
-template <int WT, int BM, int BN, int WM, int WN, int WK, int WPE>
+// GRP (MUL_MAT_ID): a column tile is an entry of the plan, its columns are
+// (expert, token) pairs with activation rows and destinations of their own.
+template <int WT, int BM, int BN, int WM, int WN, int WK, int WPE, bool GRP>
 __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) k_gemm_kq(const MatmulArgs a) {
     kernarg_prefetch<(kernarg_lines(sizeof(MatmulArgs)))>();
     constexpr int NT = 64 * WM * WN * WK, P = kq_planes<WT>(), SB = block_bytes(WT);
@@ -224,23 +48,46 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
     __shared__ __attribute__((aligned(16))) uint8_t sMin[MIN ? BM : 1][16];
     __shared__ __attribute__((aligned(16))) float sDx[BN];
     __shared__ __attribute__((aligned(16))) _Float16 sBs[MIN ? BN : 1][16];
+    __shared__ int64_t sOut[GRP ? BN : 1];  // byte offset of a column's outputs
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
     const int64_t K = a.K, nsb = K / QKK;
-    const uint32_t batches = (uint32_t)(a.ne12 * a.ne13);
+    const uint32_t batches = GRP ? 1u : (uint32_t)(a.ne12 * a.ne13);
     const uint32_t kc = batches == 1 ? blockIdx.z : blockIdx.z / batches, batch = blockIdx.z - kc * batches;
     const MmSlice sl = mm_slice(a, batch);
     const uint8_t *W = sl.w;
     const ActView act = act_view(a.act, TLH_TYPE_Q8_K, K, mm_act_rows(a));
+    const int64_t nkc = gridDim.z / batches;
     // grid x: the token tiles of a row tile next to each other (any number of rows)
-    const uint32_t ntn = (uint32_t)((a.N + BN - 1) / BN);
-    const uint32_t tm = ntn == 1 ? blockIdx.x : blockIdx.x / ntn;
+    const uint32_t ntn = (uint32_t)(GRP ? a.grp_tiles : (a.N + BN - 1) / BN);
+    const uint32_t tm = ntn == 1 ? blockIdx.x : blockIdx.x / ntn, tn = blockIdx.x - tm * ntn;
     const int64_t m_base = (int64_t)tm * BM;
-    const int64_t n_base = (int64_t)(blockIdx.x - tm * ntn) * BN, n_cols = a.N - n_base;
-    // segments: as in the q4_K / q5_K GEMM (a tile lies in one)
+    int64_t n_base = (int64_t)tn * BN, n_cols = a.N - n_base;
     int sg = 0;
     int64_t m0 = 0;
-    if (a.nseg > 0) {
+    const int32_t *pairs = nullptr;
+    if constexpr (GRP) {
+        if ((int)tn >= a.grp[0]) return;
+        const int32_t *t = a.grp + 4 + 4 * (int64_t)tn;
+        const int e = t[0];
+        n_base = 0;
+        n_cols = t[2];
+        pairs = a.grp + 4 + 4 * a.grp_tiles + t[1];
+        if (tid < BN) {
+            const uint32_t p = (uint32_t)pairs[tid < n_cols ? tid : 0], tok = p / (uint32_t)a.ne12;
+            sOut[tid] = nkc > 1 ? (int64_t)p * a.M * 4 : (int64_t)(p - tok * (uint32_t)a.ne12) * a.d_nb2 + (int64_t)tok * a.d_nb3;
+        }
+        if (e < 0) {  // no such expert: NaN
+            lds_barrier();
+            char *o = nkc > 1 ? (char *)(a.part + kc * (a.ne12 * a.ne13) * a.M) : (char *)a.dst;
+            for (int i = tid; i < BM * (int)n_cols; i += NT) {
+                const int64_t m = m_base + i % BM;
+                if (m < a.M) *(float *)(o + sOut[i / BM] + 4 * m) = __builtin_nanf("");
+            }
+            return;
+        }
+        W = a.w + (int64_t)e * a.w_nb2;
+    } else if (a.nseg > 0) {  // segments: as MatmulArgs says; a tile lies in one
         sg = (int)(m_base >= a.seg_m0[1]) + (int)(a.nseg > 2 && m_base >= a.seg_m0[2]);
         m0 = a.seg_m0[sg];
         W = a.seg_w[sg];
@@ -248,6 +95,10 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
     // activation row of the tile's column c (clamped to the last one)
     auto arow = [&](int c) -> int64_t {
         const int64_t col = c < n_cols ? c : n_cols - 1;
+        if constexpr (GRP) {
+            const uint32_t p = (uint32_t)pairs[col], tok = p / (uint32_t)a.ne12, slot = p - tok * (uint32_t)a.ne12;
+            return (int64_t)(slot % (uint32_t)a.id_b1) + a.id_b1 * (int64_t)tok;
+        }
         return a.n0 + n_base + col + a.N_total * batch;
     };
 
@@ -272,7 +123,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
         kq_u4 bs;
     };
     Regs r0, r1;  // the next first and second half
-    const int64_t nkc = gridDim.z / batches, share = (nsb + nkc - 1) / nkc;
+    const int64_t share = (nsb + nkc - 1) / nkc;
     const int64_t sb0 = kc * share, sb1 = sb0 + share < nsb ? sb0 + share : nsb;
     auto fetch = [&](auto hc, int64_t sb, Regs &r) {
         constexpr int H = decltype(hc)::value;
@@ -427,10 +278,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int k = 4 * q + e;
-                        int s = S[P - 1][j][i][k];
-                        if constexpr (WT == TLH_TYPE_Q4_K) s += S[0][j][i][k] * 8;
-                        else if constexpr (P == 2) s += S[0][j][i][k] * 256;
-                        float v = (float)s * (WT == TLH_TYPE_Q3_K ? -d : d);
+                        float v = kq_sum<WT>(S[0][j][i][k], S[P - 1][j][i][k]) * d;
                         if constexpr (MIN) v -= dmin * Mn[k];
                         acc[j][i][k] += dy[e] * v;
                     }
@@ -488,10 +336,12 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
                         acc[j][i][k] += red[(((w * WM * WN + wmn) * TN + j) * TM + i) * 1024 + 64 * k + lane];
     }
 
-    // row m of column n goes to obase + n * ostride + 4 m
+    // row m of column n goes to obase + n * ostride + 4 m (GRP: obase + sOut[n] + 4 m)
     char *obase = (char *)a.dst + sl.i12 * a.d_nb2 + sl.i13 * a.d_nb3 + a.n0 * a.d_nb1;
     int64_t ostride = a.d_nb1;
-    if (nkc > 1 || a.keep_part) {
+    if constexpr (GRP) {
+        obase = nkc > 1 ? (char *)(a.part + kc * (a.ne12 * a.ne13) * a.M) : (char *)a.dst;
+    } else if (nkc > 1 || a.keep_part) {
         obase = (char *)(a.part + (kc * batches + batch) * a.N * a.M);
         ostride = 4 * a.M;
     } else if (a.nseg > 0) {
@@ -507,7 +357,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
 #pragma unroll
                 for (int k = 0; k < 16; ++k) {
                     const int c = 32 * (wn * TN + j) + 8 * (k >> 2) + 4 * lg + (k & 3);
-                    if (c < n_cols) *(float *)(obase + (n_base + c) * ostride + 4 * m) = acc[j][i][k];
+                    if (c < n_cols)
+                        *(float *)(obase + (GRP ? sOut[c] : (n_base + c) * ostride) + 4 * m) = acc[j][i][k];
                 }
         }
     }
@@ -515,12 +366,18 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
 
 template <int WT, int BM, int BN, int WM, int WN, int WK, int WPE>
 static void launch_kq_tile(const MatmulArgs &a, int ks, hipStream_t stream) {
-    const dim3 grid((unsigned)((a.N + BN - 1) / BN * ((a.M + BM - 1) / BM)), 1u, (unsigned)(a.ne12 * a.ne13 * ks));
-    hipLaunchKernelGGL((k_gemm_kq<WT, BM, BN, WM, WN, WK, WPE>), grid, dim3(64 * WM * WN * WK), 0, stream, a);
+    const int64_t mt = (a.M + BM - 1) / BM, threads = 64 * WM * WN * WK;
+    if (a.grp) {
+        const dim3 grid((unsigned)(a.grp_tiles * mt), 1u, (unsigned)ks);
+        hipLaunchKernelGGL((k_gemm_kq<WT, BM, BN, WM, WN, WK, WPE, true>), grid, dim3(threads), 0, stream, a);
+    } else {
+        const dim3 grid((unsigned)((a.N + BN - 1) / BN * mt), 1u, (unsigned)(a.ne12 * a.ne13 * ks));
+        hipLaunchKernelGGL((k_gemm_kq<WT, BM, BN, WM, WN, WK, WPE, false>), grid, dim3(threads), 0, stream, a);
+    }
 }
 
-template <int WT> static tlh_status launch_kq(const MatmulArgs &a, int ks, hipStream_t stream) {
-    switch (gemm_kq_tile(a.N).bn) {
+template <int WT> static tlh_status launch_kq(const MatmulArgs &a, int bn, int ks, hipStream_t stream) {
+    switch (bn) {
     case 32: launch_kq_tile<WT, 64, 32, 2, 1, 2, 3>(a, ks, stream); break;
     case 64: launch_kq_tile<WT, 64, 64, 2, 2, 1, 2>(a, ks, stream); break;
     default: launch_kq_tile<WT, 128, 128, 4, 2, 1, 2>(a, ks, stream); break;
@@ -540,13 +397,13 @@ KqTile gemm_kq_tile(int64_t N) {
     return {128, 128, 1};
 }
 
-tlh_status launch_gemm_kq(const MatmulArgs &a, int ks, hipStream_t stream) {
+tlh_status launch_gemm_kq(const MatmulArgs &a, int bn, int ks, hipStream_t stream) {
     switch (a.wtype) {
-    case TLH_TYPE_Q2_K: return launch_kq<TLH_TYPE_Q2_K>(a, ks, stream);
-    case TLH_TYPE_Q3_K: return launch_kq<TLH_TYPE_Q3_K>(a, ks, stream);
-    case TLH_TYPE_Q4_K: return launch_kq<TLH_TYPE_Q4_K>(a, ks, stream);
-    case TLH_TYPE_Q5_K: return launch_kq<TLH_TYPE_Q5_K>(a, ks, stream);
-    case TLH_TYPE_Q6_K: return launch_kq<TLH_TYPE_Q6_K>(a, ks, stream);
+    case TLH_TYPE_Q2_K: return launch_kq<TLH_TYPE_Q2_K>(a, bn, ks, stream);
+    case TLH_TYPE_Q3_K: return launch_kq<TLH_TYPE_Q3_K>(a, bn, ks, stream);
+    case TLH_TYPE_Q4_K: return launch_kq<TLH_TYPE_Q4_K>(a, bn, ks, stream);
+    case TLH_TYPE_Q5_K: return launch_kq<TLH_TYPE_Q5_K>(a, bn, ks, stream);
+    case TLH_TYPE_Q6_K: return launch_kq<TLH_TYPE_Q6_K>(a, bn, ks, stream);
     default: return set_error(TLH_UNSUPPORTED, "gemm_kq: weight type %d", a.wtype);
     }
 }

@@ -75,6 +75,11 @@ struct MatmulArgs {
     // into dst + e * d_nb2 + t * d_nb3. An id outside [0, id_nas) gives NaN.
     const char *ids;
     int64_t ids_nb0, ids_nb1, id_b1, id_nas;
+    // MUL_MAT_ID through a GEMM: the plan launch_group_plan wrote -- the
+    // (expert, token) pairs sorted by expert and cut into column tiles of one
+    // expert each (GroupPlan); a column of a tile is a pair
+    const int32_t *grp;
+    int64_t grp_tiles;  // the plan's tile table entries (used ones first)
     // K-split launches leave their partials in `part` without the chunk-sum
     // launch (a consumer adds them: mul_mat_compute_keep); the k-quant GEMM does
     // so with one chunk too
@@ -209,12 +214,35 @@ tlh_status launch_partial_reduce(const MatmulArgs &a, int chunks, hipStream_t st
 // reduce_epi_check: TLH_OK when it takes a and ep
 tlh_status launch_partial_reduce_epi(const MatmulArgs &a, int chunks, const GemvEpi &ep, hipStream_t stream);
 tlh_status reduce_epi_check(const MatmulArgs &a, const GemvEpi &ep);
-// Int8-plane GEMM for k-quant weights (gemm_kq.hip), any N; ksplit as above.
-tlh_status launch_gemm_kq(const MatmulArgs &a, int ksplit, hipStream_t stream);
+// Int8-plane GEMM for k-quant weights (gemm_kq.hip), any N, in tiles of bn
+// columns (gemm_kq_tile's, or the plan's with a.grp); ksplit as above.
+tlh_status launch_gemm_kq(const MatmulArgs &a, int bn, int ksplit, hipStream_t stream);
 struct KqTile {
     int bm, bn, per_cu;  // weight rows, tokens, workgroups a CU holds
 };
 KqTile gemm_kq_tile(int64_t N);
+// MUL_MAT_ID with few pairs an expert, q4_K / q5_K (gemm_kqs.hip): column tiles
+// of 16, elements of a K chunk, chunks.
+struct KqsPlan {
+    int nt, kc_elems, zc;
+    size_t lds;
+};
+KqsPlan gemm_kqs_plan(int wtype, int64_t M, int64_t cols, int64_t K, int64_t tiles);
+tlh_status launch_gemm_kqs(const MatmulArgs &a, const KqsPlan &p, hipStream_t stream);
+// MUL_MAT_ID's plan in int32 words: [0] tiles in use, from 4 on `tiles`
+// entries {expert (-1: ids outside [0, n_as)), first pair, pairs, 0}, then the
+// pairs (e + n_used t) by expert.
+struct GroupPlan {
+    int64_t tiles;  // at most
+    int64_t bytes;
+};
+inline GroupPlan group_plan(int64_t pairs, int64_t n_as, int64_t bn) {
+    int64_t t = pairs / bn + n_as + 1;
+    if (t > pairs) t = pairs;
+    return {t, align_up(4 * (4 + 4 * t + pairs), 256)};
+}
+constexpr int64_t GROUP_MAX_EXPERTS = 4096;
+tlh_status launch_group_plan(const MatmulArgs &a, int64_t bn, int32_t *plan, hipStream_t stream);
 // K chunks of the tiled prefill GEMMs: a launch of fewer 128 x 128 tiles than
 // CUs splits K into up to 512 / tiles chunks (whole stages per chunk, at least four super-blocks /
 // sixteen q8_0 blocks each), and the bytes of its partial sums.

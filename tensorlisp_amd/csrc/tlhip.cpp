@@ -910,7 +910,8 @@ tlh_status tlh_mul_mat_noalloc(const tlh_op *op, const void *src0, const void *s
 // quantized to the vec_dot type once, then output column (e, t) is expert
 // ids[e, t]'s matrix times quantized row (e % ne11) + ne11 * t, each element
 // one vec_dot. Here every (e, t) pair is one batch slice of the int8-MFMA
-// few-column kernel, which reads the expert id on the device.
+// few-column kernel, which reads the expert id on the device; with enough
+// pairs they are grouped by expert first (mmid_groups).
 struct MulMatIdShape {
     int64_t K, M, n_as, n_used, n_tok, n_b1;
     int wtype, act_type;
@@ -966,12 +967,62 @@ static int64_t mmid_partial_bytes(const MulMatIdShape &s) {
     return align_up(gemv_mfma_partial_bytes(s.K, s.M, 1, s.n_used * s.n_tok), 256);
 }
 
+// The pairs sorted by expert and multiplied by the GEMM, a tile of columns an
+// expert, so that an expert's matrix is read once (or once per tile) instead
+// of once per pair.
+struct MulMatIdGroups {
+    bool on = false;
+    int bn = 0;        // a tile's columns
+    bool stream = false;  // the streaming form (few columns an expert)
+    KqsPlan kqs{};
+    GroupPlan plan{};
+    int ks = 1;
+    int64_t part = 0;
+    int64_t bytes = 0;  // scratch: activations, plan, partials
+};
+static MulMatIdGroups mmid_groups(const MulMatIdShape &s) {
+    MulMatIdGroups g;
+    const int64_t pairs = s.n_used * s.n_tok;
+    if (!kquant_type(s.wtype) || s.n_as < 1 || s.n_as > GROUP_MAX_EXPERTS || s.K < 256) return g;
+    const double bytes = (double)s.M * (double)(s.K / 256) * block_bytes(s.wtype);
+    const int64_t per = (pairs + s.n_as - 1) / s.n_as, used = pairs < s.n_as ? pairs : s.n_as;  // evenly chosen experts
+    // few columns and enough bytes for every CU's waves to walk: the stream
+    // (16 x 512 x 1024, 6 MB: 18 us, the tiles 11)
+    g.stream = (s.wtype == TLH_TYPE_Q4_K || s.wtype == TLH_TYPE_Q5_K) && per <= 32 && (double)used * bytes >= 32e6;
+    // A pair of its own streams its matrix at 6.4 TB/s (q2_K / q6_K: 3.4); the
+    // groups read each expert's once, the stream at 4.7 TB/s and the tiles at 2.8
+    // (q6_K 4.3), behind about 8 us of planning. Measured, pairs / groups: q4_K
+    // 8 x 14336 x 4096, 16 pairs 95 / 62 us; 32 x 2048 x 4096, 32 pairs 35 / 40;
+    // q6_K 64 x 4096 x 2048, 64 pairs 128 / 123; q5_K 16 x 512 x 1024, 128 pairs
+    // 16.2 / 16.0.
+    const bool slow = s.wtype == TLH_TYPE_Q2_K || s.wtype == TLH_TYPE_Q6_K;
+    if ((double)pairs * bytes < (slow || g.stream ? 1.25 : 2.25) * (double)s.n_as * bytes + 50e6) return g;
+    g.on = true;
+    if (g.stream) {
+        g.kqs = gemm_kqs_plan(s.wtype, s.M, per, s.K, used);
+        g.bn = 16 * g.kqs.nt;
+        g.ks = g.kqs.zc;
+    } else {
+        const KqTile t = gemm_kq_tile(per);
+        g.bn = t.bn;
+        const int64_t mt = (s.M + t.bm - 1) / t.bm, units = s.K / 256;
+        int64_t ks = 256 * t.per_cu / (used * ((per + t.bn - 1) / t.bn) * mt);
+        if (ks > units / 4) ks = units / 4;
+        g.ks = ks > 1 ? (int)(ks < 16 ? ks : 16) : 1;
+    }
+    g.plan = group_plan(pairs, s.n_as, g.bn);
+    g.part = g.ks > 1 ? align_up((int64_t)g.ks * pairs * s.M * 4, 256) : 0;
+    g.bytes = mmid_act_bytes(s) + g.plan.bytes + g.part;
+    return g;
+}
+
 tlh_status tlh_mul_mat_id_scratch_bytes(const tlh_op *op, size_t *bytes) {
     if (!bytes) return set_error(TLH_INVALID, "mul_mat_id_scratch_bytes: null pointer");
     MulMatIdShape s;
     const tlh_status st = check_mul_mat_id(op, s);
     if (st != TLH_OK) return st;
-    *bytes = (size_t)(mmid_act_bytes(s) + mmid_partial_bytes(s));
+    const int64_t need = mmid_act_bytes(s) + mmid_partial_bytes(s), grouped = mmid_groups(s).bytes;
+    *bytes = (size_t)(need > grouped ? need : grouped);
     return TLH_OK;
 }
 
@@ -1017,12 +1068,22 @@ tlh_status tlh_mul_mat_id(const tlh_op *op, const void *src0, const void *src1, 
     m.d_nb1 = d.nb[1];
     m.d_nb2 = d.nb[1];
     m.d_nb3 = d.nb[2];
-    m.part = mmid_partial_bytes(s) > 0 ? (float *)((char *)scratch + mmid_act_bytes(s)) : nullptr;
     m.ids = (const char *)ids;
     m.ids_nb0 = it.nb[0];
     m.ids_nb1 = it.nb[1];
     m.id_b1 = s.n_b1;
     m.id_nas = s.n_as;
+    const MulMatIdGroups g = mmid_groups(s);
+    if (g.on && scratch_bytes >= (size_t)g.bytes) {  // (a scratch of the pairs' form keeps that form)
+        int32_t *plan = (int32_t *)((char *)scratch + mmid_act_bytes(s));
+        m.grp = plan;
+        m.grp_tiles = g.plan.tiles;
+        m.part = g.part ? (float *)((char *)plan + g.plan.bytes) : nullptr;
+        if ((st = launch_group_plan(m, g.bn, plan, hs)) != TLH_OK) return st;
+        st = g.stream ? launch_gemm_kqs(m, g.kqs, hs) : launch_gemm_kq(m, g.bn, g.ks, hs);
+        return st != TLH_OK || g.ks == 1 ? st : launch_partial_reduce(m, g.ks, hs);
+    }
+    m.part = mmid_partial_bytes(s) > 0 ? (float *)((char *)scratch + mmid_act_bytes(s)) : nullptr;
     return launch_gemv_mfma(m, hs);
 }
 
