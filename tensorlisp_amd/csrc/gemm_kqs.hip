@@ -36,7 +36,7 @@ static size_t kqs_lds(int nt, int kc, bool min) {
 // groups in turn. The entries in use are known on the device only (experts
 // above the average take two); dealt out here they all run at once, where a
 // grid laid out for the average ran a second round (198 pairs on 8 experts, 11
-// entries: 134 -> 95 us). z: K chunks.
+// entries: 134 -> 108 us). z: K chunks.
 template <int WT, int NT>
 __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a, int kc_elems) {
     kernarg_prefetch<(kernarg_lines(sizeof(MatmulArgs) + 4))>();

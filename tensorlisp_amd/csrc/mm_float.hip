@@ -10,14 +10,13 @@
 // differs). Every weight and activation value is exact in f32, so the
 // products are too; only the accumulation order separates the two.
 //
-// One workgroup of 4 waves covers 16 weight rows x 8 src1 columns of one
-// batch slice: a wave owns 4 rows, each lane a run of K, so a wave reads its
-// rows as wide contiguous loads while the 8 columns' runs stay in registers;
-// the 32 partial sums per lane meet in DPP wave sums. Aligned rows
-// (16-byte rows and strides, K a multiple of 8) move 8 elements per lane per
-// step; any other layout runs element by element. Used for attention-shaped
-// products (the reference's attn:sdpa path, K and V views of a cache) and
-// float weight matrices; none of it is on the quantized decode path.
+// Rows of a multiple of 8 elements on 16-byte addresses and strides go to the
+// matrix cores (gemm_float.hip). The kernel here takes any other layout, element
+// by element: one workgroup of 4 waves covers 16 weight rows x 8 src1 columns of
+// one batch slice, a wave 4 rows, a lane every 64th element of K, and the 32
+// partial sums per lane meet in DPP wave sums. Used for attention-shaped
+// products (the reference's attn:sdpa path, K and V views of a cache) and float
+// weight matrices; none of it is on the quantized decode path.
 #include "kernels.hpp"
 
 namespace tlh {
@@ -43,6 +42,27 @@ __global__ void __launch_bounds__(256) k_mm_float_convert(const FloatMM f, char 
     char *orow = out + row * out_row;
     const int es = f.wtype == TLH_TYPE_F32 ? 4 : 2;
     const int xs = f.xtype == TLH_TYPE_F32 ? 4 : 2;
+    // rows of 16-byte aligned f32: 8 values a thread, stored as 16 bytes (300 rows of
+    // 4096: 8.0 us with a value a thread and 16 workgroups a row)
+    if (es == 2 && xs == 4 && (((uintptr_t)xr | (uintptr_t)orow) & 15) == 0) {
+        const int64_t full = f.K / 8;
+        for (int64_t k = blockIdx.x * 256 + threadIdx.x; k < full; k += (int64_t)gridDim.x * 256) {
+            const float4 a = ((const float4 *)xr)[2 * k], b = ((const float4 *)xr)[2 * k + 1];
+            const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            uint32_t q[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                q[i] = f.wtype == TLH_TYPE_F16 ? f2h(v[2 * i]) | (uint32_t)f2h(v[2 * i + 1]) << 16
+                                               : f32_to_bf16(v[2 * i]) | (uint32_t)f32_to_bf16(v[2 * i + 1]) << 16;
+            ((uint4 *)orow)[k] = make_uint4(q[0], q[1], q[2], q[3]);
+        }
+        const int64_t k = full * 8 + threadIdx.x;
+        if (blockIdx.x == 0 && k < f.K) {
+            const float v = as_dot(((const float *)xr)[k], f.wtype, f.xtype);
+            ((uint16_t *)orow)[k] = f.wtype == TLH_TYPE_F16 ? f2h(v) : f32_to_bf16(v);
+        }
+        return;
+    }
     for (int64_t k = blockIdx.x * 256 + threadIdx.x; k < f.K; k += (int64_t)gridDim.x * 256) {
         const float v = as_dot(ld_flt(xr + k * xs, f.xtype), f.wtype, f.xtype);
         if (es == 4) ((float *)orow)[k] = v;
@@ -71,28 +91,7 @@ __device__ __forceinline__ float wave_sum_f(float v) {
 
 constexpr int MMF_ROWS = 4, MMF_COLS = 8;  // per wave; a workgroup is 4 waves (16 rows)
 
-// 8 consecutive elements of type TY at p (16 or 32 bytes, aligned) as f32
-template <int TY> __device__ __forceinline__ void ld8(const char *p, float (&v)[8]) {
-    if constexpr (TY == TLH_TYPE_F32) {
-        const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 16);
-        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-    } else {
-        const uint4 a = *(const uint4 *)p;
-        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if constexpr (TY == TLH_TYPE_F16) {
-                v[2 * i] = h2f((uint16_t)(w[i] & 0xffff));
-                v[2 * i + 1] = h2f((uint16_t)(w[i] >> 16));
-            } else {
-                v[2 * i] = __uint_as_float(w[i] << 16);
-                v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-            }
-        }
-    }
-}
-
-template <int WT, int XT, bool VEC>
+template <int WT, int XT>
 __global__ void __launch_bounds__(256) k_mm_float(const FloatMM f) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -118,36 +117,15 @@ __global__ void __launch_bounds__(256) k_mm_float(const FloatMM f) {
     for (int r = 0; r < MMF_ROWS; ++r)
 #pragma unroll
         for (int c = 0; c < MMF_COLS; ++c) acc[r][c] = 0.0f;
-    if constexpr (VEC) {
-        for (int64_t k = 8 * (int64_t)lane; k < f.K; k += 512) {
-            float xv[MMF_COLS][8];
+    for (int64_t k = lane; k < f.K; k += 64) {
+        float xv[MMF_COLS];
 #pragma unroll
-            for (int c = 0; c < MMF_COLS; ++c) {
-                ld8<XT>(xr[c] + k * XS, xv[c]);
+        for (int c = 0; c < MMF_COLS; ++c) xv[c] = as_dot(ld_flt(xr[c] + k * XS, XT), WT, XT);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) xv[c][e] = as_dot(xv[c][e], WT, XT);
-            }
+        for (int r = 0; r < MMF_ROWS; ++r) {
+            const float wv = ld_flt(wr[r] + k * ES, WT);
 #pragma unroll
-            for (int r = 0; r < MMF_ROWS; ++r) {
-                float wv[8];
-                ld8<WT>(wr[r] + k * ES, wv);
-#pragma unroll
-                for (int c = 0; c < MMF_COLS; ++c)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[r][c] = __builtin_fmaf(wv[e], xv[c][e], acc[r][c]);
-            }
-        }
-    } else {
-        for (int64_t k = lane; k < f.K; k += 64) {
-            float xv[MMF_COLS];
-#pragma unroll
-            for (int c = 0; c < MMF_COLS; ++c) xv[c] = as_dot(ld_flt(xr[c] + k * XS, XT), WT, XT);
-#pragma unroll
-            for (int r = 0; r < MMF_ROWS; ++r) {
-                const float wv = ld_flt(wr[r] + k * ES, WT);
-#pragma unroll
-                for (int c = 0; c < MMF_COLS; ++c) acc[r][c] = __builtin_fmaf(wv, xv[c], acc[r][c]);
-            }
+            for (int c = 0; c < MMF_COLS; ++c) acc[r][c] = __builtin_fmaf(wv, xv[c], acc[r][c]);
         }
     }
     char *D = (char *)f.d + i12 * f.d_nb2 + i13 * f.d_nb3;
@@ -161,37 +139,30 @@ __global__ void __launch_bounds__(256) k_mm_float(const FloatMM f) {
         }
 }
 
-static bool aligned16(const void *p, int64_t a, int64_t b, int64_t c) {
-    return (((uintptr_t)p | (uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0;
-}
-
-template <int WT, int XT>
-static void launch_mmf(const FloatMM &f, dim3 grid, bool vec, hipStream_t s) {
-    if (vec) hipLaunchKernelGGL((k_mm_float<WT, XT, true>), grid, dim3(256), 0, s, f);
-    else hipLaunchKernelGGL((k_mm_float<WT, XT, false>), grid, dim3(256), 0, s, f);
-}
-
 tlh_status launch_mm_float(const FloatMM &f, hipStream_t stream) {
     if (f.M == 0 || f.N == 0 || f.ne12 * f.ne13 == 0) return TLH_OK;
     const int64_t gx = (f.M + 15) / 16, gy = (f.N + MMF_COLS - 1) / MMF_COLS, gz = f.ne12 * f.ne13;
     if (gx > INT32_MAX || gy > 65535 || gz > 65535) return set_error(TLH_UNSUPPORTED, "mul_mat (float): grid too large");
     const dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)gz);
-    const bool vec = f.K % 8 == 0 && aligned16(f.w, f.w_nb1, f.w_nb2, f.w_nb3) && aligned16(f.x, f.x_nb1, f.x_nb2, f.x_nb3);
+    void (*kernel)(const FloatMM);
     switch (f.wtype * 64 + f.xtype) {
-    case TLH_TYPE_F32 * 64 + TLH_TYPE_F32: launch_mmf<TLH_TYPE_F32, TLH_TYPE_F32>(f, grid, vec, stream); break;
-    case TLH_TYPE_F16 * 64 + TLH_TYPE_F32: launch_mmf<TLH_TYPE_F16, TLH_TYPE_F32>(f, grid, vec, stream); break;
-    case TLH_TYPE_F16 * 64 + TLH_TYPE_F16: launch_mmf<TLH_TYPE_F16, TLH_TYPE_F16>(f, grid, vec, stream); break;
-    case TLH_TYPE_BF16 * 64 + TLH_TYPE_F32: launch_mmf<TLH_TYPE_BF16, TLH_TYPE_F32>(f, grid, vec, stream); break;
-    case TLH_TYPE_BF16 * 64 + TLH_TYPE_BF16: launch_mmf<TLH_TYPE_BF16, TLH_TYPE_BF16>(f, grid, vec, stream); break;
+    case TLH_TYPE_F32 * 64 + TLH_TYPE_F32: kernel = k_mm_float<TLH_TYPE_F32, TLH_TYPE_F32>; break;
+    case TLH_TYPE_F16 * 64 + TLH_TYPE_F32: kernel = k_mm_float<TLH_TYPE_F16, TLH_TYPE_F32>; break;
+    case TLH_TYPE_F16 * 64 + TLH_TYPE_F16: kernel = k_mm_float<TLH_TYPE_F16, TLH_TYPE_F16>; break;
+    case TLH_TYPE_BF16 * 64 + TLH_TYPE_F32: kernel = k_mm_float<TLH_TYPE_BF16, TLH_TYPE_F32>; break;
+    case TLH_TYPE_BF16 * 64 + TLH_TYPE_BF16: kernel = k_mm_float<TLH_TYPE_BF16, TLH_TYPE_BF16>; break;
     default: return set_error(TLH_UNSUPPORTED, "mul_mat: weights %d with activations %d", f.wtype, f.xtype);
     }
+    if (gemm_float_aligned(f)) return launch_gemm_float(f, stream);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, f);
     return check_launch("mul_mat_float");
 }
 
 tlh_status launch_mm_float_convert(const FloatMM &f, void *out, int64_t out_row, hipStream_t stream) {
     const int64_t rows = f.N * f.ne12 * f.ne13;
     if (rows == 0 || f.K == 0) return TLH_OK;
-    const int64_t gx = (f.K + 255) / 256 < 64 ? (f.K + 255) / 256 : 64;
+    const int64_t per = f.wtype != TLH_TYPE_F32 && f.xtype == TLH_TYPE_F32 ? 2048 : 256;
+    const int64_t gx = (f.K + per - 1) / per < 64 ? (f.K + per - 1) / per : 64;
     const int64_t gy = rows < 65535 ? rows : 65535;
     hipLaunchKernelGGL(k_mm_float_convert, dim3((unsigned)gx, (unsigned)gy, (unsigned)((rows + gy - 1) / gy)),
                        dim3(256), 0, stream, f, (char *)out, out_row);

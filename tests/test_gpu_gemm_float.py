@@ -1,0 +1,71 @@
+"""GPU parity: the matrix-core kernels for f32 / f16 / bf16 MUL_MAT (gemm_float.hip)
+at the edges of their tiles, K remainders and dispatch, against 64-bit products.
+
+Products are exact in f32, so only the f32 sums round: with at most c additions
+in any chain (a split: the steps of one wave and 3 tree levels; a tile: 4 blocks
+of 128 bytes and then one addition per 4 blocks) an output is within
+c * 2^-24 * sum_k |w_k x_k|; K <= 2056 gives c < 16, so 1e-6 of that sum.
+"""
+from __future__ import annotations
+
+import pytest
+
+from tensorlisp_amd import native as N
+
+pytestmark = pytest.mark.gpu
+
+# M, K, N, (slices, weight slices): one row of 8; partial 16-byte chunks, blocks and
+# waves; every column tile width and its remainder; 64 x 64 tiles from 256 of them
+# (N <= 16: 512; f32: N > 32); 128 x 128 tiles from 256
+SHAPES = [(1, 8, 1, 1, 1), (33, 72, 16, 1, 1), (31, 520, 17, 3, 1), (4097, 264, 31, 1, 1), (4128, 200, 48, 1, 1),
+          (100, 1032, 49, 4, 2), (65, 2056, 5, 6, 3), (1030, 40, 1000, 1, 1), (64 * 511 + 1, 24, 9, 1, 1),
+          (16321, 136, 33, 1, 1), (63, 64, 65, 256, 128), (2049, 200, 2000, 1, 1), (129, 72, 127, 128, 128)]
+
+
+def rows(torch, t, pad):
+    """The same values in rows pad elements apart from touching."""
+    buf = torch.zeros(*t.shape[:-1], t.shape[-1] + pad, dtype=t.dtype, device=t.device)
+    buf[..., :t.shape[-1]] = t
+    return buf[..., :t.shape[-1]]
+
+
+@pytest.mark.parametrize("M,K,n,b,wb", SHAPES)
+@pytest.mark.parametrize("name", ["f32", "f16", "bf16"])
+def test_against_64_bits_and_the_general_kernel(gpu, name, M, K, n, b, wb):
+    """Aligned rows (matrix cores; one launch, and conversion + products) and rows
+    an odd number of elements apart (the element-wise kernel)."""
+    import torch
+
+    dt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[name]
+    g = torch.Generator(device="cuda").manual_seed(M * 31 + K + n)
+    w = torch.randn(1, wb, M, K, device="cuda", generator=g).to(dt)
+    x = torch.randn(1, b, n, K, device="cuda", generator=g)
+    xd = x.to(dt).double()
+    wd = w.double().repeat_interleave(b // wb, 1)
+    want = torch.matmul(xd, wd.transpose(2, 3).contiguous())
+    bound = torch.matmul(xd.abs(), wd.abs().transpose(2, 3).contiguous()) * 1e-6
+    calls = [(w, x, False), (w, x, True), (rows(torch, w, 8), rows(torch, x, 4), False), (rows(torch, w, 1), x, False),
+             (w, x.to(dt), False)]
+    for i, (ww, xx, split) in enumerate(calls):
+        y = N.mul_mat_views(ww, xx, split=split)
+        assert ((y.double() - want).abs() <= bound).all(), f"call {i}"
+
+
+@pytest.mark.parametrize("name,tiny", [("f16", 1e-7), ("bf16", 1e-39)])
+@pytest.mark.parametrize("n", [16, 77, 1040])
+def test_src1_rounds_to_nearest_even_and_subnormals_count(gpu, name, tiny, n):
+    """Through an identity matrix every output is src1 rounded to the weight
+    type, exactly: over random bits, and over subnormals of the type."""
+    import torch
+
+    dt = torch.float16 if name == "f16" else torch.bfloat16
+    K, M = 256, 1024
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randint(-2**31, 2**31 - 1, (n, K), device="cuda", generator=g, dtype=torch.int32).view(torch.float32)
+    x = torch.where(torch.isfinite(x.to(dt).float()), x, torch.ones_like(x))
+    x[::2] = torch.randn(len(x[::2]), K, device="cuda", generator=g) * tiny
+    w = torch.eye(K, device="cuda").to(dt).repeat(M // K, 1)
+    y = N.mul_mat_views(w.reshape(1, 1, M, K), x.reshape(1, 1, n, K)).reshape(n, M)
+    assert (y == x.to(dt).float().repeat(1, M // K)).all()
+    y = N.mul_mat_views((w * tiny * 3).reshape(1, 1, M, K), torch.full((1, 1, n, K), 1024.0, device="cuda"))
+    assert (y == (w * tiny * 3).float().sum(1) * 1024.0).all() and (y != 0).all()
