@@ -38,6 +38,10 @@ template <int WT, int BM, int BN, int WM, int WN, int WK, int WPE, bool GRP>
 __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) k_gemm_kq(const MatmulArgs a) {
     kernarg_prefetch<(kernarg_lines(sizeof(MatmulArgs)))>();
     constexpr int NT = 64 * WM * WN * WK, P = kq_planes<WT>(), SB = block_bytes(WT);
+    // Every 8 super-blocks the sums move to a second set, which keeps the chains of
+    // f32 additions short (q6_K K = 14336, error against 64 bits, rms over rms:
+    // 1.0e-7 -> 7.7e-8 at 115.1 -> 116.9 us). The 64-row tiles' K chunks do that.
+    constexpr bool FLUSH = BM == 128;
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32, KST = 4 / WK;
     constexpr int UPT = BM * 4 / NT, BPT = BN * 8 / NT;  // weight units, activation pieces a thread stages
     constexpr bool MIN = kq_has_min<WT>();
@@ -189,12 +193,13 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
 
     const int lr = lane & 31, lg = lane >> 5;
     kq_v16i S[P][TN][TM];
-    kq_v16f acc[TN][TM];
+    kq_v16f acc[TN][TM], tot[FLUSH ? TN : 1][FLUSH ? TM : 1];
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             acc[j][i] = (kq_v16f){};
+            if constexpr (FLUSH) tot[j][i] = (kq_v16f){};
 #pragma unroll
             for (int p = 0; p < P; ++p) S[p][j][i] = (kq_v16i){};
         }
@@ -259,7 +264,13 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
             kq_v8h mv = {};
             if constexpr (MIN) {
                 dmin = sDmin[r];
-                const kq_u2 m = *(const kq_u2 *)&sMin[r][8 * lg];
+                kq_u2 m = *(const kq_u2 *)&sMin[r][8 * lg];
+                if constexpr (WK == 2) {  // the mins of this wave's own K steps, 4 wk .. 4 wk + 3 of each
+                    // half's 8: apart, the two terms round at their own sizes and not at
+                    // their difference's (N = 32: 1.2e-7 -> 7.8e-8)
+                    m.x = wk == 0 ? m.x : 0u;
+                    m.y = wk == 1 ? m.y : 0u;
+                }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) mv[e] = (_Float16)(float)(((e < 4 ? m.x : m.y) >> (8 * (e & 3))) & 0xff);
             }
@@ -267,10 +278,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
             for (int j = 0; j < TN; ++j) {
                 const int c0 = 32 * (wn * TN + j);
                 kq_v16f Mn = {};
-                if constexpr (MIN) {
-                    if (WK == 1 || wk == 0)
-                        Mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const kq_v8h *)&sBs[c0 + lr][8 * lg], mv, (kq_v16f){}, 0, 0, 0);
-                }
+                if constexpr (MIN)
+                    Mn = __builtin_amdgcn_mfma_f32_32x32x16_f16(*(const kq_v8h *)&sBs[c0 + lr][8 * lg], mv, (kq_v16f){}, 0, 0, 0);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const float4 y4 = *(const float4 *)&sDx[c0 + 8 * q + 4 * lg];
@@ -306,8 +315,25 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
             commit(H0{}, r0);  // (past the share: read by nobody)
             fetch(H0{}, sb + 2, r0);
             if constexpr (!MIN) finalize();
+            if constexpr (FLUSH) {
+                if (((sb - sb0) & 7) == 7) {
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int i = 0; i < TM; ++i) {
+                            tot[j][i] += acc[j][i];
+                            acc[j][i] = (kq_v16f){};
+                        }
+                }
+            }
             lds_barrier();
         }
+    }
+    if constexpr (FLUSH) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int i = 0; i < TM; ++i) acc[j][i] += tot[j][i];
     }
     if constexpr (WK > 1) {
         // the K shares' sums, added in wave order through LDS
