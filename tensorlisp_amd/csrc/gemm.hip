@@ -5,26 +5,37 @@
 
 namespace tlh {
 
-int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
-    if (!has_gemm(wtype) || N <= 16) return 1;
-    constexpr int64_t CUS = 256;  // MI355X
-    int64_t ks;
+static int ksplit_of(int64_t ks, int64_t K) {
     const int64_t units = (K + 255) / 256, min_units = 4;  // units of a chunk: 256 elements
-    if (kquant_type(wtype)) {  // as many chunks as one round of workgroups holds
-        const KqTile t = gemm_kq_tile(N);
-        ks = CUS * t.per_cu / ((N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * batches);
-    } else {  // two 128 x 128 tiles a CU
-        const int64_t tiles = (N + 127) / 128 * ((M + 127) / 128) * batches;
-        if (tiles >= CUS) return 1;
-        ks = (2 * CUS + tiles - 1) / tiles;
-    }
     if (ks > units / min_units) ks = units / min_units;
     if (ks > 16) ks = 16;
     return ks > 1 ? (int)ks : 1;
 }
 
+// q8_0 / q4_0, 128 x 128 tiles: two tiles a CU
+static int ksplit_128(int64_t M, int64_t N, int64_t K, int64_t batches) {
+    constexpr int64_t CUS = 256;  // MI355X
+    const int64_t tiles = (N + 127) / 128 * ((M + 127) / 128) * batches;
+    return tiles >= CUS ? 1 : ksplit_of((2 * CUS + tiles - 1) / tiles, K);
+}
+
+int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
+    if (!has_gemm(wtype) || N <= 16) return 1;
+    constexpr int64_t CUS = 256;
+    if (!kquant_type(wtype) && N > 64) return ksplit_128(M, N, K, batches);
+    // as many chunks as one round of workgroups holds
+    const KqTile t = kquant_type(wtype) ? gemm_kq_tile(N) : gemm_q8_tile(N);
+    const int ks = ksplit_of(CUS * t.per_cu / ((N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * batches), K);
+    if (kquant_type(wtype)) return ks;
+    const int most = ksplit_128(M, N, K, batches);  // what gemm_partial_bytes has room for
+    return ks < most ? ks : most;
+}
+
 int64_t gemm_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
-    const int ks = gemm_ksplit(wtype, M, N, K, batches);
+    if (!has_gemm(wtype) || N <= 16) return 0;
+    // (q8_0 / q4_0: 128 x 128 tiles' chunks at any N, which the sizes told to
+    // callers, and so what tlh_mul_mat_noalloc refuses, have always included)
+    const int ks = kquant_type(wtype) ? gemm_ksplit(wtype, M, N, K, batches) : ksplit_128(M, N, K, batches);
     return ks > 1 ? (int64_t)ks * batches * N * M * 4 : 0;
 }
 

@@ -221,6 +221,7 @@ struct KqTile {
     int bm, bn, per_cu;  // weight rows, tokens, workgroups a CU holds
 };
 KqTile gemm_kq_tile(int64_t N);
+KqTile gemm_q8_tile(int64_t N);  // q8_0 / q4_0 (gemm_q8.hip)
 // MUL_MAT_ID with few pairs an expert, q4_K / q5_K (gemm_kqs.hip): column tiles
 // of 16, elements of a K chunk, chunks.
 struct KqsPlan {
