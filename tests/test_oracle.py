@@ -684,6 +684,7 @@ def test_float_mul_mat_against_f64(t, name):
     assert (np.abs(got - want) <= bound).all()
 
 
+@pytest.mark.skipif(ref() is None, reason="oracle/_ref (compiled reference) not built here")
 @pytest.mark.parametrize("t,name", FLOATS, ids=[n for _, n in FLOATS])
 def test_float_mul_mat_matches_reference_live(t, name):
     r = ref()
