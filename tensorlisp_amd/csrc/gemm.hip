@@ -5,8 +5,14 @@
 
 namespace tlh {
 
+int k_chunks(int64_t parts, int64_t ks) {
+    if (ks < 2) return 1;
+    const int64_t share = (parts + ks - 1) / ks;  // (the kernels' own)
+    return (int)((parts + share - 1) / share);
+}
+// at least four units of 256 elements a chunk
 static int ksplit_of(int64_t ks, int64_t K) {
-    const int64_t units = (K + 255) / 256, min_units = 4;  // units of a chunk: 256 elements
+    const int64_t units = (K + 255) / 256, min_units = 4;
     if (ks > units / min_units) ks = units / min_units;
     if (ks > 16) ks = 16;
     return ks > 1 ? (int)ks : 1;
@@ -22,13 +28,22 @@ static int ksplit_128(int64_t M, int64_t N, int64_t K, int64_t batches) {
 int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
     if (!has_gemm(wtype) || N <= 16) return 1;
     constexpr int64_t CUS = 256;
-    if (!kquant_type(wtype) && N > 64) return ksplit_128(M, N, K, batches);
+    const bool kq = kquant_type(wtype);
+    const int64_t parts = kq ? K / 256 : (K + 127) / 128;  // super-blocks, or stages of four blocks
+    if (!kq && N > 64) return k_chunks(parts, ksplit_128(M, N, K, batches));
     // as many chunks as one round of workgroups holds
-    const KqTile t = kquant_type(wtype) ? gemm_kq_tile(N) : gemm_q8_tile(N);
+    const KqTile t = kq ? gemm_kq_tile(N) : gemm_q8_tile(N);
     const int ks = ksplit_of(CUS * t.per_cu / ((N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * batches), K);
-    if (kquant_type(wtype)) return ks;
+    if (kq) return k_chunks(parts, ks);
     const int most = ksplit_128(M, N, K, batches);  // what gemm_partial_bytes has room for
-    return ks < most ? ks : most;
+    return k_chunks(parts, ks < most ? ks : most);
+}
+
+int gemm_ksplit_grouped(int64_t M, int64_t K, int64_t pairs, int64_t n_as) {
+    const int64_t per = (pairs + n_as - 1) / n_as, used = pairs < n_as ? pairs : n_as;  // evenly chosen experts
+    const KqTile t = gemm_kq_tile(per);
+    const int64_t tiles = used * ((per + t.bn - 1) / t.bn) * ((M + t.bm - 1) / t.bm);
+    return k_chunks(K / 256, ksplit_of(256 * t.per_cu / tiles, K));
 }
 
 int64_t gemm_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {

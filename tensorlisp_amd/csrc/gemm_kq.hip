@@ -81,8 +81,8 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
             const uint32_t p = (uint32_t)pairs[tid < n_cols ? tid : 0], tok = p / (uint32_t)a.ne12;
             sOut[tid] = nkc > 1 ? (int64_t)p * a.M * 4 : (int64_t)(p - tok * (uint32_t)a.ne12) * a.d_nb2 + (int64_t)tok * a.d_nb3;
         }
+        lds_barrier();  // sOut, before any use: a chunk without super-blocks meets no other barrier
         if (e < 0) {  // no such expert: NaN
-            lds_barrier();
             char *o = nkc > 1 ? (char *)(a.part + kc * (a.ne12 * a.ne13) * a.M) : (char *)a.dst;
             for (int i = tid; i < BM * (int)n_cols; i += NT) {
                 const int64_t m = m_base + i % BM;

@@ -248,6 +248,11 @@ tlh_status launch_group_plan(const MatmulArgs &a, int64_t bn, int32_t *plan, hip
 // CUs splits K into up to 512 / tiles chunks (whole stages per chunk, at least four super-blocks /
 // sixteen q8_0 blocks each), and the bytes of its partial sums.
 int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches);
+// of MUL_MAT_ID's tiles (M rows an expert, pairs on n_as experts)
+int gemm_ksplit_grouped(int64_t M, int64_t K, int64_t pairs, int64_t n_as);
+// the chunks that ks shares of ceil(parts / ks) parts of K leave with any: of 56
+// super-blocks in 9 shares of 7 the last would have none
+int k_chunks(int64_t parts, int64_t ks);
 int64_t gemm_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches);
 tlh_status launch_gemm(const MatmulArgs &a, hipStream_t stream);  // any N, from the scratch
 // k-quant GEMM that leaves its K chunks (one or more) in a.part and whose

@@ -1006,12 +1006,8 @@ static MulMatIdGroups mmid_groups(const MulMatIdShape &s) {
         g.bn = 16 * g.kqs.nt;
         g.ks = g.kqs.zc;
     } else {
-        const KqTile t = gemm_kq_tile(per);
-        g.bn = t.bn;
-        const int64_t mt = (s.M + t.bm - 1) / t.bm, units = s.K / 256;
-        int64_t ks = 256 * t.per_cu / (used * ((per + t.bn - 1) / t.bn) * mt);
-        if (ks > units / 4) ks = units / 4;
-        g.ks = ks > 1 ? (int)(ks < 16 ? ks : 16) : 1;
+        g.bn = gemm_kq_tile(per).bn;
+        g.ks = gemm_ksplit_grouped(s.M, s.K, pairs, s.n_as);
     }
     g.plan = group_plan(pairs, s.n_as, g.bn);
     g.part = g.ks > 1 ? align_up((int64_t)g.ks * pairs * s.M * 4, 256) : 0;

@@ -1,0 +1,49 @@
+"""The tiled GEMMs' splits of K (csrc/gemm.hip), read from the library on the
+CPU: no chunk may be left without a share of K, whatever the shape."""
+from __future__ import annotations
+
+import ctypes as C
+import itertools
+
+import pytest
+
+from tensorlisp_amd import native as N
+
+I64 = C.c_int64
+
+
+def fn(name, *args):
+    f = getattr(N.lib(), name)
+    f.argtypes, f.restype = list(args), C.c_int
+    return f
+
+
+def empty_chunks(parts, ks):
+    """Chunk c of ks takes parts c * share .. of ceil(parts / ks) each."""
+    return ks > 1 and -(-parts // ks) * (ks - 1) >= parts
+
+
+ROWS = (64, 448, 512, 1000, 1024, 1792, 4096, 14336, 32000)
+
+
+def test_grouped_splits_leave_no_chunk_empty():
+    """MUL_MAT_ID's tiles (448 x 14336 on 8 experts of 64 pairs each, 1792 x 14336
+    on 2: nine shares of 56 super-blocks leave the last with none)."""
+    split = fn("_ZN3tlh19gemm_ksplit_groupedEllll", I64, I64, I64, I64)
+    seen = set()
+    for M, units, n_as, per in itertools.product(ROWS, range(1, 113), (1, 2, 3, 4, 8, 64), (1, 17, 33, 64, 65, 200)):
+        ks = split(M, 256 * units, per * n_as, n_as)
+        assert ks >= 1 and not empty_chunks(units, ks), (M, 256 * units, n_as, per, ks)
+        seen.add(ks)
+    assert split(448, 14336, 512, 8) == 8 and len(seen) > 8
+
+
+@pytest.mark.parametrize("t", [N.Q8_0, N.Q4_0, N.Q2_K, N.Q4_K, N.Q6_K], ids=lambda t: N.TYPE_NAMES[t])
+def test_splits_leave_no_chunk_empty(t):
+    split = fn("_ZN3tlh11gemm_ksplitEillll", C.c_int, I64, I64, I64, I64)
+    step = N.BLOCK[t][0]
+    for M, units, n, batches in itertools.product(ROWS, range(1, 113), (17, 33, 65, 129, 300, 2048), (1, 2)):
+        for K in {256 * units, 256 * units - 224} if step == 32 else {256 * units}:
+            ks = split(t, M, n, K, batches)
+            parts = -(-K // 128) if step == 32 else units
+            assert ks >= 1 and not empty_chunks(parts, ks), (M, K, n, batches, ks)

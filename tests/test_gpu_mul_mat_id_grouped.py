@@ -4,6 +4,8 @@ gemm_kqs.hip), through the executor, against the oracle's MUL_MAT of each pair's
 expert. Bound per element as in test_gpu_gemm_kq.py."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -67,6 +69,21 @@ def test_tiles(gpu, t, n_as, per_slot):
     labels = run_case(t, M, K, n_as, used, used if per_slot else 1, tokens, 11 * n_as, columns=300,
                       bad=((3, -1), (2 * tokens - 1, n_as), (100, 1 << 30)))
     assert "group_plan" in labels, labels
+
+
+@pytest.mark.parametrize("t", [Q2_K, Q3_K, Q4_K, Q5_K, Q6_K], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("M,K,n_as,tokens,chunks", [(450, 8448, 4, 60, 7), (448, 11008, 3, 75, 9), (300, 6400, 3, 150, 5),
+                                                    (450, 7168, 4, 60, 7)], ids=["32", "64", "128", "32-even"])
+def test_tiles_with_k_chunks(gpu, t, M, K, n_as, tokens, chunks):
+    """Tiles of 32, 64 and 128 pairs over several chunks of K, all equal or the
+    last one shorter, through the partial sums: row tails, ids outside [0, n_as)."""
+    split = N.lib()._ZN3tlh19gemm_ksplit_groupedEllll
+    split.argtypes, split.restype = [C.c_int64] * 4, C.c_int
+    assert split(M, K, 2 * tokens, n_as) == chunks
+    print(f"[mul_mat_id] tiles {NAMES[t]} {n_as} x {M} x {K}, {tokens} tokens, {chunks} chunks", flush=True)
+    labels = run_case(t, M, K, n_as, 2, 2 if tokens == 75 else 1, tokens, M + K, columns=24,
+                      bad=((3, -1), (2 * tokens - 1, n_as)))
+    assert "group_plan" in labels and "gemm_kqs" not in labels, labels
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q5_K], ids=lambda t: NAMES[t])
