@@ -22,11 +22,11 @@ static int ksplit_of(int64_t ks, int64_t K) {
 static int ksplit_128(int64_t M, int64_t N, int64_t K, int64_t batches) {
     constexpr int64_t CUS = 256;  // MI355X
     const int64_t tiles = (N + 127) / 128 * ((M + 127) / 128) * batches;
-    return tiles >= CUS ? 1 : ksplit_of((2 * CUS + tiles - 1) / tiles, K);
+    return tiles == 0 || tiles >= CUS ? 1 : ksplit_of((2 * CUS + tiles - 1) / tiles, K);
 }
 
 int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
-    if (!has_gemm(wtype) || N <= 16) return 1;
+    if (!has_gemm(wtype) || N <= 16 || M == 0 || batches == 0) return 1;
     constexpr int64_t CUS = 256;
     const bool kq = kquant_type(wtype);
     const int64_t parts = kq ? K / 256 : (K + 127) / 128;  // super-blocks, or stages of four blocks

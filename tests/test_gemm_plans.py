@@ -47,3 +47,11 @@ def test_splits_leave_no_chunk_empty(t):
             ks = split(t, M, n, K, batches)
             parts = -(-K // 128) if step == 32 else units
             assert ks >= 1 and not empty_chunks(parts, ks), (M, K, n, batches, ks)
+
+
+@pytest.mark.parametrize("t", [N.Q8_0, N.Q4_0, N.Q2_K, N.Q3_K, N.Q4_K, N.Q5_K, N.Q6_K, N.Q5_0, N.F16],
+                         ids=lambda t: N.TYPE_NAMES[t])
+def test_scratch_of_no_rows(t):
+    """A MUL_MAT without weight rows has a size (it used to divide by its tiles)."""
+    for n in (1, 16, 17, 40, 300):
+        assert N.mul_mat_scratch_bytes(N.mul_mat_op(t, 0, 512, n)) > 0, n
