@@ -18,24 +18,39 @@ static int ksplit_of(int64_t ks, int64_t K) {
     return ks > 1 ? (int)ks : 1;
 }
 
-// q8_0 / q4_0, 128 x 128 tiles: two tiles a CU
-static int ksplit_128(int64_t M, int64_t N, int64_t K, int64_t batches) {
+// The chunks that the scratch sizes told to callers (and so what
+// tlh_mul_mat_noalloc refuses) have always counted, of tiles of 128 rows:
+// q8_0 / q4_0, and q4_K / q5_K up to 128 columns, two 128-column tiles a CU;
+// q4_K / q5_K above, one 256-column tile.
+static int ksplit_told(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
     constexpr int64_t CUS = 256;  // MI355X
-    const int64_t tiles = (N + 127) / 128 * ((M + 127) / 128) * batches;
-    return tiles == 0 || tiles >= CUS ? 1 : ksplit_of((2 * CUS + tiles - 1) / tiles, K);
+    const bool wide = kquant_type(wtype) && N > 128;
+    const int64_t bn = wide ? 256 : 128, tiles = (N + bn - 1) / bn * ((M + 127) / 128) * batches;
+    if (tiles == 0 || tiles >= CUS) return 1;
+    return ksplit_of(wide ? CUS / tiles : (2 * CUS + tiles - 1) / tiles, K);
 }
+static bool told_type(int wtype) { return wtype != TLH_TYPE_Q2_K && wtype != TLH_TYPE_Q3_K && wtype != TLH_TYPE_Q6_K; }
 
 int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
     if (!has_gemm(wtype) || N <= 16 || M == 0 || batches == 0) return 1;
     constexpr int64_t CUS = 256;
     const bool kq = kquant_type(wtype);
     const int64_t parts = kq ? K / 256 : (K + 127) / 128;  // super-blocks, or stages of four blocks
-    if (!kq && N > 64) return k_chunks(parts, ksplit_128(M, N, K, batches));
-    // as many chunks as one round of workgroups holds
-    const KqTile t = kq ? gemm_kq_tile(N) : gemm_q8_tile(N);
-    const int ks = ksplit_of(CUS * t.per_cu / ((N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * batches), K);
-    if (kq) return k_chunks(parts, ks);
-    const int most = ksplit_128(M, N, K, batches);  // what gemm_partial_bytes has room for
+    int64_t ks = 16;
+    if (kq || N <= 64) {  // as many chunks as one round of workgroups holds
+        const KqTile t = kq ? gemm_kq_tile(N) : gemm_q8_tile(N);
+        ks = ksplit_of(CUS * t.per_cu / ((N + t.bn - 1) / t.bn * ((M + t.bm - 1) / t.bm) * batches), K);
+    }
+    int64_t most;  // what gemm_partial_bytes has room for
+    if (told_type(wtype)) {
+        most = ksplit_told(wtype, M, N, K, batches);
+    } else {
+        // their chunks came with the tiled GEMM: no node that fitted the static
+        // scratch of tlh_mul_mat_noalloc may outgrow it by them (q6_K 512 x 14336,
+        // N = 3584: 55 MB of activations, 7 MB a chunk)
+        const int64_t room = (int64_t)TLH_NOALLOC_SCRATCH_BYTES - act_layout(TLH_TYPE_Q8_K, K, N * batches).total;
+        most = room < 0 ? ks : (room & ~(int64_t)255) / (batches * N * M * 4);
+    }
     return k_chunks(parts, ks < most ? ks : most);
 }
 
@@ -48,10 +63,11 @@ int gemm_ksplit_grouped(int64_t M, int64_t K, int64_t pairs, int64_t n_as) {
 
 int64_t gemm_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches) {
     if (!has_gemm(wtype) || N <= 16) return 0;
-    // (q8_0 / q4_0: 128 x 128 tiles' chunks at any N, which the sizes told to
-    // callers, and so what tlh_mul_mat_noalloc refuses, have always included)
-    const int ks = kquant_type(wtype) ? gemm_ksplit(wtype, M, N, K, batches) : ksplit_128(M, N, K, batches);
-    return ks > 1 ? (int64_t)ks * batches * N * M * 4 : 0;
+    const int64_t ks = told_type(wtype) ? ksplit_told(wtype, M, N, K, batches) : gemm_ksplit(wtype, M, N, K, batches);
+    const int64_t bytes = ks > 1 ? ks * batches * N * M * 4 : 0;
+    // q2_K / q3_K / q6_K: at least what their 16-column slabs took
+    const int64_t slab = told_type(wtype) ? 0 : gemv_mfma_partial_bytes(K, M, N, batches);
+    return bytes > slab ? bytes : slab;
 }
 
 tlh_status launch_gemm_epi(const MatmulArgs &a, const GemvEpi &ep, hipStream_t stream) {

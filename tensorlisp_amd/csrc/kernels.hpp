@@ -244,9 +244,10 @@ inline GroupPlan group_plan(int64_t pairs, int64_t n_as, int64_t bn) {
 }
 constexpr int64_t GROUP_MAX_EXPERTS = 4096;
 tlh_status launch_group_plan(const MatmulArgs &a, int64_t bn, int32_t *plan, hipStream_t stream);
-// K chunks of the tiled prefill GEMMs: a launch of fewer 128 x 128 tiles than
-// CUs splits K into up to 512 / tiles chunks (whole stages per chunk, at least four super-blocks /
-// sixteen q8_0 blocks each), and the bytes of its partial sums.
+// K chunks of the tiled GEMMs (at least four units of 256 elements each), where
+// the tiles alone leave CUs idle: as many as one round of workgroups holds, with
+// the tile's rows, columns and workgroups a CU (q8_0 / q4_0 above 64 columns: as
+// two rounds hold); and the bytes of the partial sums that scratch sizes count.
 int gemm_ksplit(int wtype, int64_t M, int64_t N, int64_t K, int64_t batches);
 // of MUL_MAT_ID's tiles (M rows an expert, pairs on n_as experts)
 int gemm_ksplit_grouped(int64_t M, int64_t K, int64_t pairs, int64_t n_as);

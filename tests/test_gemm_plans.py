@@ -55,3 +55,46 @@ def test_scratch_of_no_rows(t):
     """A MUL_MAT without weight rows has a size (it used to divide by its tiles)."""
     for n in (1, 16, 17, 40, 300):
         assert N.mul_mat_scratch_bytes(N.mul_mat_op(t, 0, 512, n)) > 0, n
+
+
+def align(n):
+    return -(-n // 256) * 256
+
+
+def told(t, M, K, n, batches):
+    """Scratch of a MUL_MAT with more than 16 columns: activation codes, scales
+    and sums; f16 codes and sums (q4_K, q5_K); chunks of 128-row tiles'
+    partials, or (q2_K, q3_K, q6_K) those of a 16-column slab."""
+    rows = n * batches
+    q8k = N.BLOCK[t][0] == 256
+    act = align(align(align(rows * K) + rows * (K // (256 if q8k else 32)) * 4) + rows * K // 8)
+    if t in (N.Q2_K, N.Q3_K, N.Q6_K):
+        chunks = -(-K // 4096)
+        return act + (align(chunks * batches * 16 * M * 4) if chunks > 1 else 0)
+    if q8k:
+        act += align(rows * (K + K // 16) * 2)
+    wide = q8k and n > 128
+    tiles = -(-n // (256 if wide else 128)) * -(-M // 128) * batches
+    ks = 1 if tiles >= 256 else min(256 // tiles if wide else -(-512 // tiles), -(-K // 256) // 4, 16)
+    return act + (align(ks * batches * n * M * 4) if ks > 1 else 0)
+
+
+@pytest.mark.parametrize("t", [N.Q8_0, N.Q4_0, N.Q2_K, N.Q3_K, N.Q4_K, N.Q5_K, N.Q6_K], ids=lambda t: N.TYPE_NAMES[t])
+def test_scratch_sizes(t):
+    """The sizes, and so what the static scratch takes, stay as they were before
+    the tiles and splits of the present kernels; q2_K, q3_K and q6_K, whose
+    chunks are newer, may ask for more, but not past the static scratch where
+    they fitted it. Whatever the size, the split has room in it."""
+    static = 64 << 20
+    split = fn("_ZN3tlh11gemm_ksplitEillll", C.c_int, I64, I64, I64, I64)
+    for M, K, n, batches in itertools.product((1, 64, 512, 1000, 4096, 14336, 32000), (256, 512, 4096, 5120, 14336),
+                                              (17, 32, 33, 64, 65, 128, 129, 512, 3584), (1, 2, 48, 100, 300)):
+        got = N.mul_mat_scratch_bytes(N.mul_mat_op(t, M, K, n, ne2=batches, w_ne2=1))
+        want = told(t, M, K, n, batches)
+        if t in (N.Q2_K, N.Q3_K, N.Q6_K):
+            assert got >= want and (got > static) == (want > static), (M, K, n, batches)
+        else:
+            assert got == want, (M, K, n, batches)
+        ks = split(t, M, n, K, batches)
+        act = align(align(align(n * batches * K) + n * batches * K // 64) + n * batches * K // 8)
+        assert ks == 1 or N.BLOCK[t][0] == 32 or act + ks * batches * n * M * 4 <= got, (M, K, n, batches, ks)
