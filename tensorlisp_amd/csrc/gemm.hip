@@ -70,11 +70,21 @@ int64_t gemm_partial_bytes(int wtype, int64_t M, int64_t N, int64_t K, int64_t b
     return bytes > slab ? bytes : slab;
 }
 
+// q4_K / q5_K activations of 2^31 codes and more: refused, as they have always been
+static tlh_status check_gemm_size(const MatmulArgs &a) {
+    const int64_t batches = a.ne12 * a.ne13;
+    if (kquant_type(a.wtype) && told_type(a.wtype) && (double)a.N_total * (double)batches * (double)a.K >= 2147483648.0)
+        return set_error(TLH_UNSUPPORTED, "gemm: %lld x %lld x %lld activation codes, 2^31 or more",
+                         (long long)a.N_total, (long long)batches, (long long)a.K);
+    return TLH_OK;
+}
+
 tlh_status launch_gemm_epi(const MatmulArgs &a, const GemvEpi &ep, hipStream_t stream) {
     if (!kquant_type(a.wtype) || !a.part)
         return set_error(TLH_UNSUPPORTED, "gemm: the store epilogue rides on the reduce of a k-quant GEMM");
     const int ks = gemm_ksplit(a.wtype, a.M, a.N, a.K, a.ne12 * a.ne13);
-    tlh_status st = reduce_epi_check(a, ep);
+    tlh_status st = check_gemm_size(a);
+    if (st == TLH_OK) st = reduce_epi_check(a, ep);
     if (st != TLH_OK) return st;
     MatmulArgs g = a;
     g.keep_part = 1;  // one chunk's sums go through the reduce's stores too
@@ -87,7 +97,8 @@ tlh_status launch_gemm(const MatmulArgs &a, hipStream_t stream) {
     if (has_gemm(a.wtype)) {
         const int ks = gemm_ksplit(a.wtype, a.M, a.N, a.K, batches);
         if (ks > 1 && !a.part) return set_error(TLH_INVALID, "gemm: a K split of %d needs a partials buffer", ks);
-        const tlh_status st = kquant_type(a.wtype) ? launch_gemm_kq(a, gemm_kq_tile(a.N).bn, ks, stream) : launch_gemm_q8(a, ks, stream);
+        tlh_status st = check_gemm_size(a);
+        if (st == TLH_OK) st = kquant_type(a.wtype) ? launch_gemm_kq(a, gemm_kq_tile(a.N).bn, ks, stream) : launch_gemm_q8(a, ks, stream);
         return st != TLH_OK || ks == 1 || a.keep_part ? st : launch_partial_reduce(a, ks, stream);
     }
     if (a.keep_part) return set_error(TLH_UNSUPPORTED, "gemm: no kept partials for weight type %d", a.wtype);

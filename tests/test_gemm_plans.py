@@ -98,3 +98,11 @@ def test_scratch_sizes(t):
         ks = split(t, M, n, K, batches)
         act = align(align(align(n * batches * K) + n * batches * K // 64) + n * batches * K // 8)
         assert ks == 1 or N.BLOCK[t][0] == 32 or act + ks * batches * n * M * 4 <= got, (M, K, n, batches, ks)
+
+
+@pytest.mark.parametrize("t", [N.Q4_K, N.Q5_K], ids=lambda t: N.TYPE_NAMES[t])
+def test_2_to_the_31_activation_codes_are_refused(t):
+    """Before anything is launched (the pointers here are never followed)."""
+    op = N.mul_mat_op(t, 64, 4096, 1 << 19)
+    st = N.lib().tlh_mul_mat_compute(C.byref(op), C.c_void_p(256), C.c_void_p(256), C.c_size_t(1 << 40), C.c_void_p(256), None)
+    assert N.STATUS[st] == "UNSUPPORTED" and b"2^31" in N.lib().tlh_last_error()
