@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(64 * WM * WN * WK) __attribute__((amdgpu_waves
 template <int WT, int BM, int BN, int WM, int WN, int WK, int WPE>
 static void launch_kq_tile(const MatmulArgs &a, int ks, hipStream_t stream) {
     const int64_t mt = (a.M + BM - 1) / BM, threads = 64 * WM * WN * WK;
-    if (a.grp) {
+    if (a.ids) {
         const dim3 grid((unsigned)(a.grp_tiles * mt), 1u, (unsigned)ks);
         hipLaunchKernelGGL((k_gemm_kq<WT, BM, BN, WM, WN, WK, WPE, true>), grid, dim3(threads), 0, stream, a);
     } else {

@@ -63,7 +63,17 @@ struct MatmulArgs {
     const uint8_t *seg_w[3];
     int64_t seg_w_nb1[3];
     float *seg_dst[3];
-    int64_t seg_m0[4];
+    union {
+        int64_t seg_m0[4];
+        // MUL_MAT_ID (ids != null, no segments) through a GEMM: the plan
+        // launch_group_plan wrote -- the (expert, token) pairs sorted by expert and
+        // cut into column tiles of one expert each (GroupPlan); a column of a tile
+        // is a pair.
+        struct {
+            const int32_t *grp;
+            int64_t grp_tiles;  // the plan's tile table entries (used ones first)
+        };
+    };
     // the few-column MFMA kernel also takes segments (N <= 16, one K chunk,
     // segment row counts multiples of 16, one weight row stride): segment s's
     // outputs go to seg_dst[s] + column * seg_d_nb1[s] bytes
@@ -75,16 +85,15 @@ struct MatmulArgs {
     // into dst + e * d_nb2 + t * d_nb3. An id outside [0, id_nas) gives NaN.
     const char *ids;
     int64_t ids_nb0, ids_nb1, id_b1, id_nas;
-    // MUL_MAT_ID through a GEMM: the plan launch_group_plan wrote -- the
-    // (expert, token) pairs sorted by expert and cut into column tiles of one
-    // expert each (GroupPlan); a column of a tile is a pair
-    const int32_t *grp;
-    int64_t grp_tiles;  // the plan's tile table entries (used ones first)
     // K-split launches leave their partials in `part` without the chunk-sum
     // launch (a consumer adds them: mul_mat_compute_keep); the k-quant GEMM does
     // so with one chunk too
     int keep_part;
 };
+// 16 bytes more of arguments cost every launch of these kernels 0.1 .. 0.2 us
+// (q5_1 512 x 13056, N = 1000, 63 slabs of two launches: 1204 -> 1216 us; q5_0
+// 2432 x 1792, N = 61, four slabs: 36.5 -> 37.2)
+static_assert(sizeof(MatmulArgs) <= 344, "kernel arguments");
 
 // Batch slice z of a MUL_MAT launch: i12 = z % ne12, i13 = z / ne12 and the
 // weight matrix it reads (broadcast by r2 / r3). Slice 0 -- the only one of a
@@ -215,7 +224,7 @@ tlh_status launch_partial_reduce(const MatmulArgs &a, int chunks, hipStream_t st
 tlh_status launch_partial_reduce_epi(const MatmulArgs &a, int chunks, const GemvEpi &ep, hipStream_t stream);
 tlh_status reduce_epi_check(const MatmulArgs &a, const GemvEpi &ep);
 // Int8-plane GEMM for k-quant weights (gemm_kq.hip), any N, in tiles of bn
-// columns (gemm_kq_tile's, or the plan's with a.grp); ksplit as above.
+// columns (gemm_kq_tile's, or the plan's with a.ids); ksplit as above.
 tlh_status launch_gemm_kq(const MatmulArgs &a, int bn, int ksplit, hipStream_t stream);
 struct KqTile {
     int bm, bn, per_cu;  // weight rows, tokens, workgroups a CU holds
