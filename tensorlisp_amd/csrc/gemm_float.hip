@@ -14,8 +14,8 @@
 //
 // Lane-wise fused multiply-adds on the vector ALUs, which these kernels
 // replaced, took, in us (f32 src1): f16 4096 x 4096 N = 1 23.4 -> 8.4, N = 16
-// 36.4 -> 9.3, N = 77 107 -> 17.0, N = 512 586 -> 44; f16 8192 x 8192 N = 512
-// 2699 -> 118; bf16 1024 x 1024 N = 64 13.2 -> 7.4; f32 4096 x 4096 N = 77
+// 36.4 -> 9.3, N = 77 107 -> 17.0, N = 512 586 -> 46; f16 8192 x 8192 N = 512
+// 2699 -> 151; bf16 1024 x 1024 N = 64 13.2 -> 7.4; f32 4096 x 4096 N = 77
 // 144 -> 37, N = 1 22.1 -> 20.6; f32 512 x 128, N = 512, 32 slices 397 -> 38.
 // Error against 64 bits, rms over rms, f16 4096 x 4096: 1.5e-7 -> 1.0e-7
 // (split), 1.3e-7 (tiles); f32 1.6e-7 -> 1.4e-7; K = 8192: 2.0e-7 -> 1.5e-7.
@@ -206,13 +206,16 @@ __global__ void __launch_bounds__(64 * KW) k_mmf_split(const FloatMM f, int mt, 
 // both operands staged through two LDS buffers of 128 bytes a row, 16-byte
 // chunk c of row r at c ^ (r & 7) (reads of 8 rows touch all banks once). D
 // blocks' loads fly while one is multiplied (64 x 64 tiles, f16 4096 x 4096, N =
-// 200: D = 1 / 2 / 3 / 4 48 / 40 / 35 / 33 us). Every FLUSH blocks the sums move
+// 200: D = 1 / 2 / 3 / 4 48 / 40 / 35 / 33 us). XF: f32 src1 rounded on its way
+// to LDS; its loads are twice as many, so fewer blocks fly (D = 2 / 3 / 4 39 / 36 /
+// 50 us: four leave no registers). Every FLUSH blocks the sums move
 // to a second set, which keeps the chains of f32 additions short. 8192 x 8192, N
 // = 512: 583 TFLOP/s, bound by LDS reads (64 x 64 a wave: as long as its MFMAs)
 // and by one round of tiles on the chip.
-template <int TY, int B, int WPE, int D>
+template <int TY, int B, int WPE, int D, bool XF>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) k_mmf_tile(const FloatMM f, int mt, int nt) {
-    constexpr int F = B / 32, LD = B / 16, FLUSH = TY == TLH_TYPE_F32 ? 1 : 4;  // fragments a side, loads a thread and block
+    constexpr int F = B / 32, LD = B / 16, FLUSH = TY == TLH_TYPE_F32 ? 1 : 4;  // fragments a side, rows a thread and block
+    constexpr int LQ = LD + (XF ? B / 32 : 0);  // 16-byte loads (f32 src1: two a row)
     __shared__ __align__(16) char lds[2][2 * B * 128];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
     const MmfView v = batch_view(f);
@@ -229,11 +232,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE)))
         const int64_t at = (isw ? m0 : n0) + t, end = isw ? f.M : f.N;
         src[i] = (isw ? v.w : v.x) + (at < end ? at : end - 1) * (isw ? f.w_nb1 : f.x_nb1);
     }
-    u4 q[D][LD];
-    auto fetch = [&](u4 (&q)[LD], int64_t off) {
+    u4 q[D][LQ];
+    auto fetch = [&](u4 (&q)[LQ], int64_t off) {
         const int64_t at = off + 16 * c < kb ? off + 16 * c : kb - 16;
 #pragma unroll
-        for (int i = 0; i < LD; ++i) q[i] = *(const u4 *)(src[i] + at);
+        for (int i = 0; i < LD; ++i) {
+            if (XF && i >= B / 32) {
+                q[i] = *(const u4 *)(src[i] + 2 * at);
+                q[i + B / 32] = *(const u4 *)(src[i] + 2 * at + 16);
+            } else {
+                q[i] = *(const u4 *)(src[i] + at);
+            }
+        }
     };
     const int st = lr * 128 + ((c ^ (lr & 7)) * 16);
     const int wm = (wave & 1) * (B / 2), wn = (wave >> 1) * (B / 2);
@@ -244,9 +254,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE)))
 #pragma unroll
         for (int j = 0; j < F; ++j) acc[i][j] = (f4)(0.0f), sum[i][j] = (f4)(0.0f);
     int buf = 0, chain = 0;
-    auto block = [&](u4 (&q)[LD], int64_t off) {
+    auto block = [&](u4 (&q)[LQ], int64_t off) {
         char *L = lds[buf];
         buf ^= 1;
+        if constexpr (XF) {
+#pragma unroll
+            for (int i = B / 32; i < LD; ++i) q[i] = round8<TY>(q[i], q[i + B / 32]);
+        }
         if (off + 128 > kb && off + 16 * c >= kb) {
 #pragma unroll
             for (int i = 0; i < LD; ++i) q[i] = (u4)(0u);
@@ -321,7 +335,7 @@ bool gemm_float_aligned(const FloatMM &f) {
 // N = 64 128 tiles, 31 against 22). Up to 16 columns two a CU (32768 x 4096:
 // 46 against 56); f32, which would multiply 64 columns at an eighth of the
 // rate, above 32 columns only (4096 x 4096, N = 32: 106 against 23).
-bool gemm_float_tiled(const FloatMM &f) {
+static bool gemm_float_tiled(const FloatMM &f) {
     const int64_t t = tiles2(f, 64, 64);
     return f.wtype == TLH_TYPE_F32 ? f.N > 32 && t >= 256 : t >= (f.N > 16 ? 256 : 512);
 }
@@ -339,19 +353,25 @@ template <int TY, int NT, int D> static void launch_split(const FloatMM &f, hipS
     hipLaunchKernelGGL((k_mmf_split<TY, NT, D, false>), grid, dim3(64 * KW), bytes, s, f, mt, nt);
 }
 
-template <int TY, int B, int WPE, int D> static void launch_tile(const FloatMM &f, hipStream_t s) {
+template <int TY, int B, int WPE, int D, int DX = D> static void launch_tile(const FloatMM &f, hipStream_t s) {
     const int mt = (int)tiles(f.M, B), nt = (int)tiles(f.N, B);
     const dim3 grid((unsigned)(mt * nt), (unsigned)(f.ne12 * f.ne13));
-    hipLaunchKernelGGL((k_mmf_tile<TY, B, WPE, D>), grid, dim3(256), 0, s, f, mt, nt);
+    if constexpr (TY != TLH_TYPE_F32) {
+        if (f.xtype != TY) {
+            hipLaunchKernelGGL((k_mmf_tile<TY, B, WPE, DX, true>), grid, dim3(256), 0, s, f, mt, nt);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_mmf_tile<TY, B, WPE, D, false>), grid, dim3(256), 0, s, f, mt, nt);
 }
 
 template <int TY> static void launch_ty(const FloatMM &f, hipStream_t s) {
-    if (f.xtype == f.wtype && gemm_float_tiled(f)) {
+    if (gemm_float_tiled(f)) {
         // 128 x 128 tiles once there is one a CU (f16 8192 x 8192, N = 512: 118 us,
         // with 64 x 64 tiles 127; 4096 x 4096, N = 512, half as many: 65 against 44);
         // f32 is bound by its MFMAs (8192 x 4096, N = 512: 320 against 292)
-        if (TY != TLH_TYPE_F32 && tiles2(f, 128, 128) >= 256) launch_tile<TY, 128, 2, 2>(f, s);
-        else launch_tile<TY, 64, 3, 4>(f, s);
+        if (TY != TLH_TYPE_F32 && tiles2(f, 128, 128) >= 256) launch_tile<TY, 128, 2, 2, 1>(f, s);
+        else launch_tile<TY, 64, 3, 4, 3>(f, s);
         return;
     }
     // Columns a workgroup: a CU's time goes with the rows it reads (32 of W,

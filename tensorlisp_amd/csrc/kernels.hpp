@@ -371,10 +371,8 @@ struct FloatMM {
     int64_t M, K, N, ne12, ne13, r2, r3;
 };
 tlh_status launch_mm_float(const FloatMM &f, hipStream_t stream);
-// the same on the matrix cores (gemm_float.hip), for aligned operands; tiled:
-// enough outputs that x rows are better converted to the weight type first
+// the same on the matrix cores (gemm_float.hip), for aligned operands
 bool gemm_float_aligned(const FloatMM &f);
-bool gemm_float_tiled(const FloatMM &f);
 tlh_status launch_gemm_float(const FloatMM &f, hipStream_t stream);
 // x rows -> contiguous rows of the weight type at out (out_row bytes apart)
 tlh_status launch_mm_float_convert(const FloatMM &f, void *out, int64_t out_row, hipStream_t stream);

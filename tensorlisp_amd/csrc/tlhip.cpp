@@ -762,13 +762,10 @@ tlh_status tlh_mul_mat(const tlh_op *op, const void *src0, const void *src1, voi
     if ((st = mm_check_scratch(s, scratch, scratch_bytes)) != TLH_OK) return st;
     const hipStream_t hs = (hipStream_t)stream;
     const tlh_tensor &b = op->t[1];
-    if (s.flt) {  // one launch that rounds src1 as it reads it, or the rounded rows first for many outputs
+    if (s.flt) {  // one launch that rounds src1 as it reads it; the scratch is left alone
         if ((uintptr_t)src0 % float_size(s.wtype) || (uintptr_t)src1 % float_size(b.ty) || ((uintptr_t)dst & 3))
             return set_error(TLH_INVALID, "mul_mat: misaligned src0, src1 or dst");
-        const FloatMM f = float_mm(op, s, src0, src1, b.ty, b.nb, dst);
-        if (b.ty == s.wtype || !gemm_float_aligned(f) || !gemm_float_tiled(f)) return launch_mm_float(f, hs);
-        if ((st = launch_mm_float_convert(f, scratch, mm_float_row(s), hs)) != TLH_OK) return st;
-        return mm_compute(op, s, src0, scratch, dst, hs);
+        return launch_mm_float(float_mm(op, s, src0, src1, b.ty, b.nb, dst), hs);
     }
     // Decode with a small activation: the GEMV quantizes src1 itself (one launch).
     const bool packed = b.nb[2] == b.nb[1] * s.N && b.nb[3] == b.nb[2] * s.ne12;

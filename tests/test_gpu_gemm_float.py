@@ -69,3 +69,26 @@ def test_src1_rounds_to_nearest_even_and_subnormals_count(gpu, name, tiny, n):
     assert (y == x.to(dt).float().repeat(1, M // K)).all()
     y = N.mul_mat_views((w * tiny * 3).reshape(1, 1, M, K), torch.full((1, 1, n, K), 1024.0, device="cuda"))
     assert (y == (w * tiny * 3).float().sum(1) * 1024.0).all() and (y != 0).all()
+
+
+@pytest.mark.parametrize("M,K,n", [(64, 512, 1), (1024, 4096, 77), (4096, 256, 300), (16384, 64, 130)])
+@pytest.mark.parametrize("name", ["f32", "f16", "bf16"])
+def test_one_call_leaves_the_scratch_alone(gpu, name, M, K, n):
+    """tlh_mul_mat with float weights is one launch that reads f32 src1: a scratch
+    that another stream's products, or a quantize before it, use stays as it is."""
+    import torch
+
+    dt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[name]
+    g = torch.Generator(device="cuda").manual_seed(n)
+    w = torch.randn(M, K, device="cuda", generator=g).to(dt)
+    x, other = torch.randn(2, n, K, device="cuda", generator=g)
+    mm = N.MulMat({"f32": N.F32, "f16": N.F16, "bf16": N.BF16}[name], M, K, n)
+    y, z = torch.empty(2, n, M, device="cuda")
+    mm.quantize(x)
+    before = mm.scratch.clone()
+    mm(w, other, y)
+    assert torch.equal(mm.scratch, before)
+    mm.compute(w, z)
+    mm(w, x, y)
+    bound = (x.to(dt).double().abs() @ w.double().abs().T) * 2e-6
+    assert ((y.double() - z.double()).abs() <= bound).all()
