@@ -96,6 +96,27 @@ def test_stream(gpu, t, M, K, n_as, tokens):
     assert "gemm_kqs" in labels, labels
 
 
+class Stream(C.Structure):
+    _fields_ = [("nt", C.c_int), ("kc_elems", C.c_int), ("zc", C.c_int), ("lds", C.c_size_t)]
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("M,K,n_as,tokens", [(64, 8704, 162, 190), (40, 4096, 520, 640)])
+def test_stream_walks_several_entries(gpu, t, M, K, n_as, tokens):
+    """More plan entries than the stream's grid has workgroups (256 over the K
+    chunks): each fills its LDS again for the next one."""
+    plan = N.lib()._ZN3tlh13gemm_kqs_planEillll
+    plan.argtypes, plan.restype = [C.c_int] + [C.c_int64] * 4, Stream
+    pairs = 2 * tokens
+    p = plan(t, M, -(-pairs // n_as), K, min(pairs, n_as))
+    ids = np.random.default_rng(M + tokens).integers(0, n_as - 1, (tokens, 2))  # (run_case's)
+    entries = (-(-np.bincount(ids.reshape(-1)) // (16 * p.nt))).sum()
+    print(f"[mul_mat_id] stream {NAMES[t]} {n_as} x {M} x {K}, {tokens} tokens, {entries} entries, {p.zc} chunks", flush=True)
+    assert entries > 256 // p.zc
+    labels = run_case(t, M, K, n_as, 2, 2 if K == 4096 else 1, tokens, M + tokens, columns=120, bad=((5, n_as + 3),))
+    assert "gemm_kqs" in labels, labels
+
+
 def test_plan_of_many_experts(gpu):
     """More experts than the plan's workgroup has threads."""
     labels = run_case(Q4_K, 40, 256, 1500, 4, 4, 4200, 3, columns=200, bad=((0, 1500),))
