@@ -19,6 +19,8 @@ typedef int kq_v4i __attribute__((ext_vector_type(4)));
 typedef int kq_v16i __attribute__((ext_vector_type(16)));
 typedef float kq_v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 kq_v8h __attribute__((ext_vector_type(8)));
+typedef float kq_v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 kq_v4h __attribute__((ext_vector_type(4)));
 typedef uint32_t kq_u4 __attribute__((ext_vector_type(4)));  // (plain vectors: a struct of them stays in registers)
 typedef uint32_t kq_u2 __attribute__((ext_vector_type(2)));
 typedef unsigned short kq_u16x2 __attribute__((ext_vector_type(2)));
