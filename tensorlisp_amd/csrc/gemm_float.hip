@@ -13,10 +13,10 @@
 // and CU (f16 4096 x 4096, N = 77: 24 us against 16).
 //
 // Lane-wise fused multiply-adds on the vector ALUs, which these kernels
-// replaced, took, in us (f32 src1): f16 4096 x 4096 N = 1 23.4 -> 8.6, N = 16
-// 36.4 -> 9.4, N = 77 107 -> 17.0, N = 512 586 -> 51; f16 8192 x 8192 N = 512
+// replaced, took, in us (f32 src1): f16 4096 x 4096 N = 1 23.4 -> 7.2, N = 16
+// 36.4 -> 7.6, N = 77 107 -> 17.0, N = 512 586 -> 51; f16 8192 x 8192 N = 512
 // 2699 -> 134; bf16 1024 x 1024 N = 64 13.2 -> 7.4; f32 4096 x 4096 N = 77
-// 141 -> 39, N = 1 22.1 -> 21.4; f32 512 x 128, N = 512, 32 slices 397 -> 45.
+// 141 -> 39, N = 1 22.1 -> 17.4; f32 512 x 128, N = 512, 32 slices 397 -> 45.
 //
 // Sums. An MFMA rounds several times on its way through K (once a k in f32, once
 // every 8 in f16 / bf16), so a chain of them is as inexact as one of that many
@@ -425,7 +425,11 @@ template <int TY> static void launch_ty(const FloatMM &f, hipStream_t s) {
         if (cost <= least) least = cost, best = nt;
     }
     if (f.N <= 16 || best == 1) {
-        launch_split<TY, 2, 1, 2>(f, s);
+        // 16 rows a workgroup while 32 would leave half of the CUs without one: f32 777
+        // x 4096, N = 1 16.2 -> 11.8 us (25 -> 49 workgroups; the lane-wise kernel, 49 of
+        // 4 waves, 14.0), f16 4096 x 4096, N = 16 9.4 -> 7.6 (128 -> 256)
+        if (tiles2(f, 32, 16) <= 128) launch_split<TY, 1, 1, 2>(f, s);
+        else launch_split<TY, 2, 1, 2>(f, s);
     } else if (best == 2) {
         launch_split<TY, 2, 2, 1>(f, s);
     } else {

@@ -2,9 +2,10 @@
 at the edges of their tiles, K remainders and dispatch, against 64-bit products.
 
 Products are exact in f32, so only the f32 sums round: with at most c additions
-in any chain (a split: the steps of one wave and 3 tree levels; a tile: 4 blocks
-of 128 bytes and then one addition per 4 blocks) an output is within
-c * 2^-24 * sum_k |w_k x_k|; K <= 2056 gives c < 16, so 1e-6 of that sum.
+on any product's way (an MFMA's own; a split: a wave's blocks of 128 bytes by
+fours and 3 tree levels; a tile: blocks by levels of two or four) an output is within
+c * 2^-24 * sum_k |w_k x_k|; K <= 2056 gives c < 16, so 1e-6 of that sum (f32: 19,
+if all of them rounded one way).
 """
 from __future__ import annotations
 
@@ -15,11 +16,13 @@ from tensorlisp_amd import native as N
 pytestmark = pytest.mark.gpu
 
 # M, K, N, (slices, weight slices): one row of 8; partial 16-byte chunks, blocks and
-# waves; every column tile width and its remainder; 64 x 64 tiles from 256 of them
-# (N <= 16: 512; f32: N > 32); 128 x 128 tiles from 256
+# waves; every column tile width and its remainder, 16 rows to 128 tiles of 32 and 32
+# above; 64 x 64 tiles from 256 of them (N <= 16: 512; f32: N > 32); 128 x 128 tiles
+# from 256 (bf16: K > 1024)
 SHAPES = [(1, 8, 1, 1, 1), (33, 72, 16, 1, 1), (31, 520, 17, 3, 1), (4097, 264, 31, 1, 1), (4128, 200, 48, 1, 1),
           (100, 1032, 49, 4, 2), (65, 2056, 5, 6, 3), (1030, 40, 1000, 1, 1), (64 * 511 + 1, 24, 9, 1, 1),
-          (16321, 136, 33, 1, 1), (63, 64, 65, 256, 128), (2049, 200, 2000, 1, 1), (129, 72, 127, 128, 128)]
+          (4129, 72, 9, 1, 1), (16321, 136, 33, 1, 1), (63, 64, 65, 256, 128), (2049, 200, 2000, 1, 1), (129, 72, 127, 128, 128),
+          (2049, 1032, 2000, 1, 1)]
 
 
 def rows(torch, t, pad):
