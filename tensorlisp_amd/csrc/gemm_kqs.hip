@@ -11,9 +11,12 @@
 // (kq_unit.hpp), so a lane loads its unit straight from the row, scales it and
 // multiplies. The activation codes of the workgroup's columns go to LDS once
 // (one barrier), then each wave walks its 16-row groups on its own, two
-// super-blocks of loads ahead. Eight q4_K experts of 14336 x 4096 (264 MB):
-// 32 pairs 101 -> 56 us (4.7 TB/s), 198 pairs 117 -> 70 us against the LDS
-// tiles. Not for q6_K: its 2-byte aligned units take seven loads a super-block
+// super-blocks of loads ahead. Eight q4_K experts of 14336 x 4096 (264 MB), the
+// kernel alone against the LDS tiles: 32 pairs 101 -> 60 us (4.4 TB/s), 198 evenly
+// dealt pairs 117 -> 68 us; as a router deals them (55 to 4 an expert) 94 us, since
+// experts above 32 pairs take two plan entries and their matrix is read twice (11
+// entries, 363 MB), and the blocks of an entry leave its last round part empty.
+// The quantize and the plan before it take 5 us each. Not for q6_K: its 2-byte aligned units take seven loads a super-block
 // (64 experts of 4096 x 2048, 128 pairs: 128 us, the tiles 101 us).
 #include "kq_unit.hpp"
 
@@ -35,8 +38,8 @@ static size_t kqs_lds(int nt, int kc, bool min) {
 // pairs of an expert each): the workers of an entry take its blocks of NW row
 // groups in turn. The entries in use are known on the device only (experts
 // above the average take two); dealt out here they all run at once, where a
-// grid laid out for the average ran a second round (198 pairs on 8 experts, 11
-// entries: 134 -> 108 us). z: K chunks.
+// grid laid out for the average ran a second round (the whole call, 198 pairs on
+// 8 experts, 11 entries: 134 -> 108 us). z: K chunks.
 template <int WT, int NT>
 __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a, int kc_elems) {
     kernarg_prefetch<(kernarg_lines(sizeof(MatmulArgs) + 4))>();
@@ -141,7 +144,12 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             kq_fetch<WT, H>(p + (int64_t)sb * SB, g, r);
         };
         kq_v4i S[P][NT];
-        kqs_v4f acc[NT];
+        // One column tile: every 4 super-blocks acc moves to tot, so that the f32 chains
+        // stay short (K = 8704 in one chunk, error against 64 bits: 1.16e-7 in one chain, 8.6e-8
+        // now, a pair of its own 1.12e-7). Two have no registers for it and at most
+        // 17 super-blocks a chunk (9.3e-8).
+        constexpr bool FLUSH = NT == 1;
+        kqs_v4f acc[NT], tot = {};
         auto multiply = [&](auto hc, int sb, const KqUnit<WT> &r) {
             constexpr int H = decltype(hc)::value;
             uint32_t o[2][2][4];
@@ -222,7 +230,16 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             multiply(H1{}, sb, u1);
             finalize(sb, u1);
             fetch(H1{}, sb + 2, u1, wrow, wnext, wnext2);
-            if (++sb < nsb) return;
+            if (++sb < nsb) {
+                if constexpr (FLUSH) {
+                    if ((sb & 3) == 0) {
+                        tot += acc[0];
+                        acc[0] = (kqs_v4f){};
+                    }
+                }
+                return;
+            }
+            if constexpr (FLUSH) acc[0] += tot;
             const int64_t m = (b * NW + wave) * 16 + lr;
             if (m < a.M) {
 #pragma unroll
@@ -236,6 +253,7 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             }
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[j] = (kqs_v4f){};
+            if constexpr (FLUSH) tot = (kqs_v4f){};
             sb = 0;
             b += workers;
             wrow = wnext;

@@ -108,20 +108,11 @@ def q8_K_codes(x):
     return np.ascontiguousarray(b[:, :, :4]).view(np.float32)[:, :, 0], b[:, :, 4:260].copy().view(np.int8).reshape(n, K)
 
 
-@pytest.mark.parametrize("t", [Q3_K, Q4_K, Q5_K, Q6_K], ids=lambda t: NAMES[t])
-@pytest.mark.parametrize("copies,K,n", [(1, 512, 20), (1, 512, 40), (1, 4096, 32), (28, 14336, 32), (28, 14336, 48), (63, 4096, 64), (8, 4096, 256)])
-def test_sums_are_as_exact_as_short_chains(gpu, t, copies, K, n):
-    """The f32 sums' error against 64 bits, root mean square over many outputs, is
-    that of each super-block's term formed in its three or four roundings and
-    added in chains of four, the chains' sums after one another: one chain over K
-    = 14336 is 1.3 times as far off, K steps of one super-block finished apart
-    1.08 times. 5% for chance (16384 outputs and more: 0.6% standard deviation)."""
-    import torch
-
-    rows = 512 if n < 100 else 64
-    w = synth.random_blocks(t, K + n, rows, K)
-    x = synth.normal(n, (n, K))
-    bb = N.BLOCK[t][1]
+def short_chains(t, w, K, x, length=4):
+    """(x @ w.T of the op's codes in 64 bits, the same in f32: each super-block's
+    term formed in its three or four roundings and added in chains of `length`,
+    the chains' sums after one another)."""
+    rows, n, bb = w.shape[0], x.shape[0], N.BLOCK[t][1]
     parts = []  # the weights' scale part and min part, each exact in f32
     for drop in ((2, 4), (0, 2)):
         b = w.reshape(-1, bb).copy()
@@ -136,15 +127,34 @@ def test_sums_are_as_exact_as_short_chains(gpu, t, copies, K, n):
         s = slice(256 * sb, 256 * sb + 256)
         q, dy = q8[:, s].astype(np.float64), d8[:, sb, None].astype(np.float64)
         a = q @ parts[0][:, s].T
-        m = q @ parts[1][:, s].T if t in (Q4_K, Q5_K) else 0.0
+        m = q @ parts[1][:, s].T if t in (Q4_K, Q5_K) else np.zeros_like(a)
         exact += dy * (a + m)
-        chain = (chain + dy * (a.astype(f32) + m).astype(f32)).astype(f32)
-        if sb % 4 == 3 or sb == K // 256 - 1:
+        v = (a + m.astype(f32)).astype(f32)  # (a fused multiply-add)
+        chain = (chain + dy * v).astype(f32)
+        if (sb + 1) % length == 0 or sb == K // 256 - 1:
             total, chain = total + chain, np.zeros_like(chain)
+    return exact, total
+
+
+def check_sums(got, exact, total, what):
+    """got's error, root mean square over the outputs, is total's. 5% for chance
+    (8192 outputs and more: 0.8% standard deviation)."""
+    rms = lambda e: np.sqrt(np.mean(e ** 2) / np.mean(exact ** 2))  # noqa: E731
+    print(f"{what}: {rms(got - exact):.3e}, short chains {rms(total - exact):.3e}", flush=True)
+    assert rms(got - exact) <= 1.05 * rms(total - exact)
+
+
+@pytest.mark.parametrize("t", [Q3_K, Q4_K, Q5_K, Q6_K], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("copies,K,n", [(1, 512, 20), (1, 512, 40), (1, 4096, 32), (28, 14336, 32), (28, 14336, 48), (63, 4096, 64), (8, 4096, 256)])
+def test_sums_are_as_exact_as_short_chains(gpu, t, copies, K, n):
+    """One chain over K = 14336 is 1.3 times as far off, K steps of one super-block
+    finished apart 1.08 times."""
+    import torch
+
+    rows = 512 if n < 100 else 64
+    w, x = synth.random_blocks(t, K + n, rows, K), synth.normal(n, (n, K))
     M = copies * rows
     y = N.mul_mat(t, dev(np.tile(w, (copies, 1))), M, K, dev(x))
     torch.cuda.synchronize()
     got = y.cpu().numpy().reshape(n, copies, rows)[:, -1].astype(np.float64)
-    rms = lambda e: np.sqrt(np.mean(e ** 2) / np.mean(exact ** 2))  # noqa: E731
-    print(f"[gemm_kq] {NAMES[t]} {M}x{K} n={n}: {rms(got - exact):.3e}, short chains {rms(total - exact):.3e}", flush=True)
-    assert rms(got - exact) <= 1.05 * rms(total - exact)
+    check_sums(got, *short_chains(t, w, K, x), f"[gemm_kq] {NAMES[t]} {M}x{K} n={n}")

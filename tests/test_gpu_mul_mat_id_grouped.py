@@ -13,7 +13,7 @@ from refs import NAMES, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, oracle
 from tensorlisp_amd import graph as G
 from tensorlisp_amd import native as N
 from tensorlisp_amd import synth
-from test_gpu_gemm_kq import bound, dev
+from test_gpu_gemm_kq import bound, check_sums, dev, short_chains
 
 pytestmark = pytest.mark.gpu
 
@@ -115,6 +115,33 @@ def test_stream_walks_several_entries(gpu, t, M, K, n_as, tokens):
     assert entries > 256 // p.zc
     labels = run_case(t, M, K, n_as, 2, 2 if K == 4096 else 1, tokens, M + tokens, columns=120, bad=((5, n_as + 3),))
     assert "gemm_kqs" in labels, labels
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("copies,K,tokens", [(28, 8704, 16), (28, 4096, 32), (8, 8704, 60)])
+def test_stream_sums_are_as_exact_as_short_chains(gpu, t, copies, K, tokens):
+    """One column tile, 34 super-blocks in one chunk (one chain of them is 1.3 times
+    as far off), and two, whose chunks of 17 are one chain each."""
+    import torch
+
+    rows, n_as = 512, 8
+    w, x = synth.random_blocks(t, K, rows, K), synth.normal(tokens, (tokens, 1, K))
+    M = copies * rows
+    op = N.TlhOp()
+    op.t[0], op.t[1] = N.ggml_tensor(t, [K, M, n_as]), N.ggml_tensor(N.F32, [K, 1, tokens])
+    op.t[2], op.t[4] = N.ggml_tensor(N.I32, [2, tokens]), N.ggml_tensor(N.F32, [M, 2, tokens])
+    need = C.c_size_t()
+    N.check(N.lib().tlh_mul_mat_id_scratch_bytes(C.byref(op), C.byref(need)))
+    scratch = torch.empty(need.value + 256, dtype=torch.uint8, device="cuda")
+    W, X = dev(w).repeat(n_as * copies, 1), dev(x)  # every expert the same rows
+    ids = torch.arange(2 * tokens, dtype=torch.int32, device="cuda") % n_as
+    y = torch.empty((tokens, 2, M), device="cuda")
+    N.check(N.lib().tlh_mul_mat_id(C.byref(op), N._ptr(W), N._ptr(X), N._ptr(ids), N._ptr(y),
+                                   C.c_void_p(scratch.data_ptr() + -scratch.data_ptr() % 256), need, N._stream(None)))
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(tokens, 2, copies, rows)[:, 1, -1].astype(np.float64)
+    exact, total = short_chains(t, w, K, x[:, 0], 17 if tokens == 60 else 4)
+    check_sums(got, exact, total, f"[mul_mat_id] stream {NAMES[t]} {n_as} x {M} x {K}, {tokens} tokens")
 
 
 def test_plan_of_many_experts(gpu):
