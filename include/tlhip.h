@@ -174,8 +174,12 @@ tlh_status tlh_mul_mat_compute(const tlh_op *op, const void *src0, const void *s
  * t[4] = dst f32 [M, n_used, n_tokens]. dst[:, e, t] = as[:, :, ids[e, t]] times
  * b row (e % n_b1, t), each element the CPU's vec_dot of the quantized row
  * (so within the MUL_MAT tolerance of the CPU backend). An id outside
- * [0, n_as) yields NaN in its column (the CPU backend aborts there). Decode
- * oriented: each (expert, token) pair streams its expert's matrix once. */
+ * [0, n_as) yields NaN in its column (the CPU backend aborts there). With few
+ * (expert, token) pairs each streams its expert's matrix once. With many and
+ * k-quant weights they are sorted by expert on the device first, and an expert's
+ * matrix is read once for a tile of its pairs; that takes the whole scratch of
+ * tlh_mul_mat_id_scratch_bytes. A smaller one that holds the quantized rows (and
+ * for K > 4096 their K-chunk sums) is taken too, with a matrix read a pair. */
 tlh_status tlh_mul_mat_id_scratch_bytes(const tlh_op *op, size_t *bytes);
 tlh_status tlh_mul_mat_id(const tlh_op *op, const void *src0, const void *src1, const void *ids, void *dst,
                           void *scratch, size_t scratch_bytes, void *stream);

@@ -22,17 +22,12 @@
 
 namespace tlh {
 
-typedef float kqs_v4f __attribute__((ext_vector_type(4)));
-typedef _Float16 kqs_v4h __attribute__((ext_vector_type(4)));
-
 constexpr int KQS_WAVES = 16;
 
 // LDS of kc elements of nt * 16 columns: codes [col][kc], scales [col][kc / 256],
 // bsums as f16 [col][kc / 16 + 8] (the pad spreads the columns over the banks)
 constexpr int kqs_bs_row(int kc) { return kc / 16 + 8; }
-static size_t kqs_lds(int nt, int kc, bool min) {
-    return (size_t)16 * nt * (kc + kc / 64 + (min ? 2 * kqs_bs_row(kc) : 0) + 16);
-}
+static size_t kqs_lds(int nt, int kc) { return (size_t)16 * nt * (kc + kc / 64 + 2 * kqs_bs_row(kc) + 16); }
 
 // Grid x: about a workgroup a CU, dealt out over the plan's entries (up to 16 NT
 // pairs of an expert each): the workers of an entry take its blocks of NW row
@@ -44,7 +39,7 @@ template <int WT, int NT>
 __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a, int kc_elems) {
     kernarg_prefetch<(kernarg_lines(sizeof(MatmulArgs) + 4))>();
     constexpr int P = kq_planes<WT>(), SB = block_bytes(WT), BN = 16 * NT, NW = KQS_WAVES;
-    constexpr bool MIN = kq_has_min<WT>();
+    static_assert(WT == TLH_TYPE_Q4_K || WT == TLH_TYPE_Q5_K, "types with eight mins");
     extern __shared__ __attribute__((aligned(16))) int8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, g = lane >> 4;
@@ -104,14 +99,12 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             for (int k = 0; k < CPW; ++k) {
                 const int col = wave + NW * k;
                 for (int i = lane; i < nsb; i += 64) sDx[i * BN + col] = act.d[sRow[col] * nsb_all + sb_first + i];
-                if constexpr (MIN) {
-                    for (int i = lane; i < 2 * nsb; i += 64) {  // 8 bsums
-                        const kq_u4 b = *(const kq_u4 *)(act.bsums + sRow[col] * (K / 16) + (int64_t)sb_first * 16 + 8 * i);
-                        kq_v8h h;
+                for (int i = lane; i < 2 * nsb; i += 64) {  // 8 bsums
+                    const kq_u4 b = *(const kq_u4 *)(act.bsums + sRow[col] * (K / 16) + (int64_t)sb_first * 16 + 8 * i);
+                    kq_v8h h;
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) h[e] = (_Float16)(float)(int16_t)(b[e >> 1] >> (16 * (e & 1)));
-                        *(kq_v8h *)(sBs + col * bs_row + 8 * i) = h;
-                    }
+                    for (int e = 0; e < 8; ++e) h[e] = (_Float16)(float)(int16_t)(b[e >> 1] >> (16 * (e & 1)));
+                    *(kq_v8h *)(sBs + col * bs_row + 8 * i) = h;
                 }
             }
         }
@@ -149,7 +142,7 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
         // now, a pair of its own 1.12e-7). Two have no registers for it and at most
         // 17 super-blocks a chunk (9.3e-8).
         constexpr bool FLUSH = NT == 1;
-        kqs_v4f acc[NT], tot = {};
+        kq_v4f acc[NT], tot = {};
         auto multiply = [&](auto hc, int sb, const KqUnit<WT> &r) {
             constexpr int H = decltype(hc)::value;
             uint32_t o[2][2][4];
@@ -174,31 +167,20 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             float d, dmin;
             uint32_t mn[4];
             kq_row_meta<WT>(r, d, dmin, mn);
-            kqs_v4h mv = {};
-            if constexpr (MIN) {  // the mins of bsums 4 g .. 4 g + 3
-                uint32_t m;
-                if constexpr (WT == TLH_TYPE_Q2_K) {
-                    const uint32_t lo = g & 1 ? mn[1] : mn[0], hi = g & 1 ? mn[3] : mn[2];
-                    m = g & 2 ? hi : lo;
-                } else {
-                    const uint32_t w = (g & 2 ? mn[1] : mn[0]) >> (16 * (g & 1));
-                    m = __builtin_amdgcn_perm(0u, w, 0x01010000u);
-                }
+            kq_v4h mv;  // the mins of bsums 4 g .. 4 g + 3
+            const uint32_t m = __builtin_amdgcn_perm(0u, (g & 2 ? mn[1] : mn[0]) >> (16 * (g & 1)), 0x01010000u);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) mv[e] = (_Float16)(float)((m >> (8 * e)) & 0xff);
-            }
+            for (int e = 0; e < 4; ++e) mv[e] = (_Float16)(float)((m >> (8 * e)) & 0xff);
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                kqs_v4f Mn = {};
-                if constexpr (MIN)
-                    Mn = __builtin_amdgcn_mfma_f32_16x16x16f16(*(const kqs_v4h *)(sBs + (16 * j + lr) * bs_row + 16 * sb + 4 * g), mv,
-                                                              (kqs_v4f){}, 0, 0, 0);
+                const kq_v4f Mn = __builtin_amdgcn_mfma_f32_16x16x16f16(
+                    *(const kq_v4h *)(sBs + (16 * j + lr) * bs_row + 16 * sb + 4 * g), mv, (kq_v4f){}, 0, 0, 0);
                 const float4 y4 = *(const float4 *)(sDx + sb * BN + 16 * j + 4 * g);
                 const float dy[4] = {y4.x, y4.y, y4.z, y4.w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float v = kq_sum<WT>(S[0][j][e], S[P - 1][j][e]) * d;
-                    if constexpr (MIN) v -= dmin * Mn[e];
+                    v -= dmin * Mn[e];
                     acc[j][e] += dy[e] * v;
                 }
 #pragma unroll
@@ -217,7 +199,7 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
         }
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            acc[j] = (kqs_v4f){};
+            acc[j] = (kq_v4f){};
 #pragma unroll
             for (int p = 0; p < P; ++p) S[p][j] = (kq_v4i){};
         }
@@ -234,7 +216,7 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
                 if constexpr (FLUSH) {
                     if ((sb & 3) == 0) {
                         tot += acc[0];
-                        acc[0] = (kqs_v4f){};
+                        acc[0] = (kq_v4f){};
                     }
                 }
                 return;
@@ -252,8 +234,8 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
                     }
             }
 #pragma unroll
-            for (int j = 0; j < NT; ++j) acc[j] = (kqs_v4f){};
-            if constexpr (FLUSH) tot = (kqs_v4f){};
+            for (int j = 0; j < NT; ++j) acc[j] = (kq_v4f){};
+            if constexpr (FLUSH) tot = (kq_v4f){};
             sb = 0;
             b += workers;
             wrow = wnext;
@@ -274,20 +256,19 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
 // 8 experts of 14336 x 4096 117 us with one) and K chunks zc: of what fits LDS,
 // and enough that the blocks of row groups of `tiles` entries reach every CU
 // (8 experts of 3000 x 8192, 16 pairs: 64 us with one chunk).
-KqsPlan gemm_kqs_plan(int wtype, int64_t M, int64_t cols, int64_t K, int64_t tiles) {
+KqsPlan gemm_kqs_plan(int64_t M, int64_t cols, int64_t K, int64_t tiles) {
     constexpr int64_t LDS = 160 * 1024;
     KqsPlan p{};
     p.nt = cols <= 8 ? 1 : 2;
-    const bool min = wtype == TLH_TYPE_Q4_K || wtype == TLH_TYPE_Q5_K;
     const int64_t nsb = K / 256, blocks = ((M + 15) / 16 + KQS_WAVES - 1) / KQS_WAVES * tiles;
     int64_t fill = (256 + blocks - 1) / blocks;
     if (fill > nsb / 4) fill = nsb / 4;
     for (p.zc = fill > 1 ? (int)fill : 1;; ++p.zc) {
         p.kc_elems = (int)((nsb + p.zc - 1) / p.zc * 256);
-        if ((int64_t)kqs_lds(p.nt, p.kc_elems, min) <= LDS) break;
+        if ((int64_t)kqs_lds(p.nt, p.kc_elems) <= LDS) break;
     }
     p.zc = (int)((nsb + p.kc_elems / 256 - 1) / (p.kc_elems / 256));  // no empty chunk
-    p.lds = kqs_lds(p.nt, p.kc_elems, min);
+    p.lds = kqs_lds(p.nt, p.kc_elems);
     return p;
 }
 

@@ -237,7 +237,7 @@ struct KqsPlan {
     int nt, kc_elems, zc;
     size_t lds;
 };
-KqsPlan gemm_kqs_plan(int wtype, int64_t M, int64_t cols, int64_t K, int64_t tiles);
+KqsPlan gemm_kqs_plan(int64_t M, int64_t cols, int64_t K, int64_t tiles);
 tlh_status launch_gemm_kqs(const MatmulArgs &a, const KqsPlan &p, hipStream_t stream);
 // MUL_MAT_ID's plan in int32 words: [0] tiles in use, from 4 on `tiles`
 // entries {expert (-1: ids outside [0, n_as)), first pair, pairs, 0}, then the

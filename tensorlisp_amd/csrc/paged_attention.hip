@@ -523,8 +523,8 @@ tlh_status launch_paged_attention(const tlh_paged_attention_args &a, void *scrat
     float *s = (float *)scratch;
     if (qo && (!counters || !qo->out || !paged_attention_quantize_ok(a, qo->type) ||
                qo->rows < a.num_seqs))
-        return set_error(TLH_UNSUPPORTED, "paged_attention: the merge quantizes whole q8_K blocks of heads, "
-                                          "one launch, no f16 codes");
+        return set_error(TLH_UNSUPPORTED, "paged_attention: the merge quantizes whole q8_K blocks of heads "
+                                          "of all sequences, in one launch");
     switch (a.head_size) {
     case 64: launch_pa1<64>(a, s, stream, out32, counters, qo); break;
     case 80: launch_pa1<80>(a, s, stream, out32, counters, qo); break;

@@ -538,7 +538,7 @@ static MatmulArgs mm_args(const tlh_op *op, const MulMatShape &s, const void *sr
     return m;
 }
 
-// Phase 2: the products from the scratch, N <= 8 -> GEMV, else GEMM.
+// Phase 2: the products from the scratch, N <= 16 -> GEMV, else GEMM.
 static tlh_status mm_compute(const tlh_op *op, const MulMatShape &s, const void *src0, const void *scratch,
                              void *dst, hipStream_t hs) {
     if (((uintptr_t)src0 & 1) || ((uintptr_t)dst & 3))
@@ -999,7 +999,7 @@ static MulMatIdGroups mmid_groups(const MulMatIdShape &s) {
     if ((double)pairs * bytes < (slow || g.stream ? 1.25 : 2.25) * (double)s.n_as * bytes + 50e6) return g;
     g.on = true;
     if (g.stream) {
-        g.kqs = gemm_kqs_plan(s.wtype, s.M, per, s.K, used);
+        g.kqs = gemm_kqs_plan(s.M, per, s.K, used);
         g.bn = 16 * g.kqs.nt;
         g.ks = g.kqs.zc;
     } else {

@@ -105,10 +105,10 @@ class Stream(C.Structure):
 def test_stream_walks_several_entries(gpu, t, M, K, n_as, tokens):
     """More plan entries than the stream's grid has workgroups (256 over the K
     chunks): each fills its LDS again for the next one."""
-    plan = N.lib()._ZN3tlh13gemm_kqs_planEillll
-    plan.argtypes, plan.restype = [C.c_int] + [C.c_int64] * 4, Stream
+    plan = N.lib()._ZN3tlh13gemm_kqs_planEllll
+    plan.argtypes, plan.restype = [C.c_int64] * 4, Stream
     pairs = 2 * tokens
-    p = plan(t, M, -(-pairs // n_as), K, min(pairs, n_as))
+    p = plan(M, -(-pairs // n_as), K, min(pairs, n_as))
     ids = np.random.default_rng(M + tokens).integers(0, n_as - 1, (tokens, 2))  # (run_case's)
     entries = (-(-np.bincount(ids.reshape(-1)) // (16 * p.nt))).sum()
     print(f"[mul_mat_id] stream {NAMES[t]} {n_as} x {M} x {K}, {tokens} tokens, {entries} entries, {p.zc} chunks", flush=True)
