@@ -55,11 +55,6 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
     kernarg_prefetch<(kernarg_lines(sizeof(MatmulArgs)))>();
     constexpr int NT = 64 * WM * WN, P = kq_planes<WT>(), SB = block_bytes(WT);
     using Tile = KqTileTypes<MT>;
-    // Every FLUSH super-blocks the sums move to a second set, which keeps the chains
-    // of f32 additions short. Error against 64 bits, rms over rms, none / 8 / 4:
-    // q4_K 14336 x 14336, N = 48 1.10e-7 / 8.6e-8 / 8.5e-8; 14336 x 4096, N = 64
-    // 7.6e-8 / 7.6e-8 / 7.2e-8; in time, 8 and 4 are alike.
-    constexpr int FLUSH = 4;
     constexpr int TM = BM / WM / MT, TN = BN / WN / MT, KST = MT / 8, NR = MT * MT / 64;  // tiles a wave, K steps a stage, results a lane
     constexpr int UPT = BM * 4 / NT, BPT = BN * 8 / NT;  // weight units, activation pieces a thread stages
     constexpr bool MIN = kq_has_min<WT>();
@@ -317,32 +312,50 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
         commit(H0{}, r0);
         fetch(H0{}, sb0 + 1, r0);
         lds_barrier();
-        for (int64_t sb = sb0; sb < sb1; ++sb) {
-            multiply(H0{});
-            commit(H1{}, r1);
-            fetch(H1{}, sb + 1, r1);
-            lds_barrier();
-            multiply(H1{});
-            if constexpr (MIN) finalize();
-            commit(H0{}, r0);  // (past the share: read by nobody)
-            fetch(H0{}, sb + 2, r0);
-            if constexpr (!MIN) finalize();
-            if ((sb - sb0) % FLUSH == FLUSH - 1) {
+        // Every 4 super-blocks the sums move to a second set (8 in long chunks), which
+        // keeps the chains of f32 additions short. Error against 64 bits, rms over rms,
+        // never / 8 / 4: q4_K 14336 x 14336, N = 48 1.10e-7 / 8.6e-8 / 8.5e-8, N = 512 (one
+        // chunk of 56) - / 8.8e-8 / 9.5e-8; 14336 x 4096, N = 64 7.6e-8 / 7.6e-8 / 7.2e-8; 4096 x
+        // 5632, 75 pairs an expert - / 7.85e-8 / 7.91e-8. In time, 8 and 4 are alike.
+        const int every = share > 20 ? 8 : 4;
+        auto flush = [&]() {
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) {
-                        tot[j][i] += acc[j][i];
-                        acc[j][i] = (typename Tile::F){};
-                    }
+                for (int i = 0; i < TM; ++i) {
+                    tot[j][i] += acc[j][i];
+                    acc[j][i] = (typename Tile::F){};
+                }
+        };
+        // The 64-row tiles run to a flush and back; one inside their loop, as in the
+        // 128 x 128 tiles, splits its schedule (q6_K 14336 x 4096, N = 64: 32.7 against 34.2
+        // us; 128 x 128 the other way round, N = 512: 126 against 110).
+        constexpr bool NEST = BM == 64;
+        int64_t sb = sb0;
+        auto upto = [&](int64_t end) {
+            for (; sb < end; ++sb) {
+                multiply(H0{});
+                commit(H1{}, r1);
+                fetch(H1{}, sb + 1, r1);
+                lds_barrier();
+                multiply(H1{});
+                if constexpr (MIN) finalize();
+                commit(H0{}, r0);  // (past the share: read by nobody)
+                fetch(H0{}, sb + 2, r0);
+                if constexpr (!MIN) finalize();
+                if constexpr (!NEST) {
+                    if (((int)(sb - sb0) & (every - 1)) == every - 1) flush();
+                }
+                lds_barrier();
             }
-            lds_barrier();
+            flush();
+        };
+        if constexpr (NEST) {
+            while (sb < sb1) upto(sb + every < sb1 ? sb + every : sb1);
+        } else {
+            upto(sb1);
         }
     }
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int i = 0; i < TM; ++i) acc[j][i] += tot[j][i];
 
     // row m of column n goes to obase + n * ostride + 4 m (GRP: obase + sOut[n] + 4 m)
     char *obase = (char *)a.dst + sl.i12 * a.d_nb2 + sl.i13 * a.d_nb3 + a.n0 * a.d_nb1;
@@ -366,7 +379,7 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
                 for (int k = 0; k < NR; ++k) {
                     const int c = MT * (wn * TN + j) + 8 * (k >> 2) + 4 * lg + (k & 3);
                     if (c < n_cols)
-                        *(float *)(obase + (GRP ? sOut[c] : (n_base + c) * ostride) + 4 * m) = acc[j][i][k];
+                        *(float *)(obase + (GRP ? sOut[c] : (n_base + c) * ostride) + 4 * m) = tot[j][i][k];
                 }
         }
     }
