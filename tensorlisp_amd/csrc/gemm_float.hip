@@ -14,19 +14,19 @@
 //
 // Lane-wise fused multiply-adds on the vector ALUs, which these kernels
 // replaced, took, in us (f32 src1): f16 4096 x 4096 N = 1 23.4 -> 7.2, N = 16
-// 36.4 -> 7.6, N = 77 107 -> 17.0, N = 512 586 -> 51; f16 8192 x 8192 N = 512
-// 2699 -> 134; bf16 1024 x 1024 N = 64 13.2 -> 7.4; f32 4096 x 4096 N = 77
+// 36.4 -> 7.6, N = 77 107 -> 16.7, N = 512 586 -> 49; f16 8192 x 8192 N = 512
+// 2699 -> 124; bf16 1024 x 1024 N = 64 13.2 -> 7.4; f32 4096 x 4096 N = 77
 // 141 -> 39, N = 1 22.1 -> 17.4; f32 512 x 128, N = 512, 32 slices 397 -> 45.
 //
 // Sums. An MFMA rounds several times on its way through K (once a k in f32, once
 // every 8 in f16 / bf16), so a chain of them is as inexact as one of that many
-// additions. Here a chain is one MFMA (f32: two), the chains of a 128-byte block
-// are added to each other, and blocks by levels of a few (the kernels say how
-// many). Error against 64 bits, rms over rms, with 64 lanes' sums / chains of
-// eight MFMAs / now: bf16 8192 x 256 5.5e-8 / 8.6e-8 / 5.5e-8, K = 4096 8.4e-8 /
-// 1.15e-7 / 8.1e-8; f16 K = 256 7.6e-8 / 1.05e-7 / 6.6e-8; f32 K = 4096 1.6e-7 /
-// 2.3e-7 / 1.0e-7. It costs 3 to 15% of the time (f16 4096 x 4096, N = 512 48 ->
-// 51 us, N = 77 16.5 -> 17.0; f32 N = 256 109 -> 124).
+// additions. Here a chain is one MFMA (f32, and f16 in the tiles: two), the chains
+// of a 128-byte block are added to each other, and blocks by levels of a few (the
+// kernels say how many: only as many as each type needs). Error against 64 bits,
+// rms over rms, with 64 lanes' sums / chains of eight MFMAs / now: bf16 8192 x 256
+// 5.5e-8 / 8.6e-8 / 5.5e-8, K = 4096 8.4e-8 / 1.15e-7 / 8.1e-8; f16 K = 256 7.6e-8
+// / 1.05e-7 / 7.0e-8; f32 K = 4096 1.6e-7 / 2.3e-7 / 1.0e-7. In us, chains of eight
+// and now: f16 4096 x 4096, N = 512 48 / 49, bf16 46 / 49; f32 N = 256 109 / 124.
 #include "kernels.hpp"
 
 namespace tlh {
@@ -38,22 +38,28 @@ typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
-// A fragment pair's product; f32 in two chains of two MFMAs (in one of four K =
-// 256 is at 9.2e-8 instead of 8.1e-8, in four 4096 x 4096, N = 256 takes 136 us
-// instead of 124)
-template <int TY> __device__ __forceinline__ f4 mma(u4 a, u4 b) {
-    const f4 zero = (f4)(0.0f);
+// A fragment pair's product, f16 / bf16 on top of c; f32 by itself, in two chains of
+// two MFMAs (in one of four K = 256 is at 9.2e-8 instead of 8.1e-8, in four 4096 x
+// 4096, N = 256 takes 136 us instead of 124)
+template <int TY> __device__ __forceinline__ f4 mma(u4 a, u4 b, f4 c = (f4)(0.0f)) {
     if constexpr (TY == TLH_TYPE_F16) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), zero, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
     } else if constexpr (TY == TLH_TYPE_BF16) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), zero, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
     } else {
         const f4 af = __builtin_bit_cast(f4, a), bf = __builtin_bit_cast(f4, b);
         f4 t[2];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) t[e >> 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[e], bf[e], e & 1 ? t[e >> 1] : zero, 0, 0, 0);
+        for (int e = 0; e < 4; ++e)
+            t[e >> 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[e], bf[e], e & 1 ? t[e >> 1] : (f4)(0.0f), 0, 0, 0);
         return t[0] + t[1];
     }
+}
+
+// a tile's 128-byte block: f16 in one chain (two MFMAs)
+template <int TY> __device__ __forceinline__ f4 mma2(u4 a0, u4 b0, u4 a1, u4 b1) {
+    if constexpr (TY == TLH_TYPE_F16) return mma<TY>(a1, b1, mma<TY>(a0, b0));
+    else return mma<TY>(a0, b0) + mma<TY>(a1, b1);
 }
 
 // eight f32 values of src1 -> the weight type, to nearest even (the CPU's conversion)
@@ -106,13 +112,16 @@ __device__ __forceinline__ MmfView batch_view(const FloatMM &f) {
 // 128-byte blocks (wave w: blocks w, w + KW, ...), so that the chip is full from
 // 256 x 16 MR rows on whatever N is. The waves share no operand: each turns its
 // blocks into fragments in LDS of its own, without a barrier, adds its blocks'
-// sums by fours, and the waves' sums meet in a tree at the end. XF: f32 src1
+// sums by fours (f16, whose products are the longest, all in one chain: K = 4096
+// 1.0e-7 and 16.4 us at 4096 x 4096, N = 77, by fours 8.6e-8 and 17.0; 64 lanes
+// 1.5e-7), and the waves' sums meet in a tree at the end. XF: f32 src1
 // rounded to the weight type as it arrives. Bound by what a CU takes in: f16 4096
 // x 4096, N = 77: 131 KB of W rows and 786 KB of f32 X rows each in about 13 us;
 // 8192 x 8192, N = 1: 5.0 TB/s of weights.
 constexpr int KW = 8;
 template <int TY, int MR, int NT, int D, bool XF>
 __global__ void __launch_bounds__(64 * KW) k_mmf_split(const FloatMM f, int mt, int nt) {
+    constexpr bool LEVELS = TY != TLH_TYPE_F16;
     constexpr int R = 16 * (MR + NT), LD = R / 8;  // rows of a block, rows a lane loads
     constexpr int LQ = LD + (XF ? 2 * NT : 0);   // 16-byte loads (f32 src1: two a row)
     extern __shared__ __align__(16) char lds[];  // [KW] blocks, then part[KW][16 NT][16 MR]
@@ -175,12 +184,13 @@ __global__ void __launch_bounds__(64 * KW) k_mmf_split(const FloatMM f, int mt, 
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
                     const f4 p = mma<TY>(a[i], a[MR + j]);
-                    if (s == 0) t[i][j] = p;
+                    if (!LEVELS) acc[i][j] += p;
+                    else if (s == 0) t[i][j] = p;
                     else acc[i][j] += t[i][j] + p;
                 }
         }
         __builtin_amdgcn_wave_barrier();
-        if ((++chain & 3) == 0) {
+        if (LEVELS && (++chain & 3) == 0) {
 #pragma unroll
             for (int i = 0; i < MR; ++i)
 #pragma unroll
@@ -231,13 +241,13 @@ __global__ void __launch_bounds__(64 * KW) k_mmf_split(const FloatMM f, int mt, 
 // 7) (reads of 8 rows touch all banks once). D blocks' loads fly while one is
 // multiplied (64 x 64 tiles, f16 4096 x 4096, N = 200: D = 1 / 2 / 3 / 4 48 / 40 /
 // 35 / 33 us). XF: f32 src1 rounded on its way to LDS. The blocks' sums go up LV
-// levels, each the sum of RAD of the one below and the last of all the rest: by
-// fours; by twos for f32, and for bf16 with K <= 1024, whose products are so short
-// that 64 lanes' first sums were exact (K = 1000: 7.0e-8 by fours, 6.7e-8 by twos,
-// 6.8e-8 the lanes). 128 x 128 tiles have eight waves, since four would hold three
-// levels of 64 results each (f16 8192 x 8192, N = 512: 191 against 134 us; with
-// one level 109). 8192 x 8192, N = 512: 510 TFLOP/s, bound by LDS reads and by one
-// round of tiles on the chip.
+// levels, each the sum of RAD of the one below and the last of all the rest: f16 two
+// of eights; bf16 three of fours, and to K = 1024 five of twos, since its products
+// are so short that 64 lanes' first sums were exact (K = 1000: 7.0e-8 by fours,
+// 6.7e-8 by twos, 6.8e-8 the lanes); f32 by twos. 128 x 128 tiles have eight waves,
+// since four would hold levels of 64 results each (f16 8192 x 8192, N = 512: 390
+// against 124 us, without levels 109 on converted rows). 8192 x 8192, N = 512: 555
+// TFLOP/s, bound by LDS reads and by one round of tiles on the chip.
 template <int TY, int B, int WM, int WN, int RAD, int LV, int D, bool XF>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2))) k_mmf_tile(const FloatMM f, int mt, int nt) {
     constexpr int FM = B / WM / 16, FN = B / WN / 16;  // fragments of a wave
@@ -307,7 +317,7 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) lev[0][i][j] += mma<TY>(a[0][i], b[0][j]) + mma<TY>(a[1][i], b[1][j]);
+            for (int j = 0; j < FN; ++j) lev[0][i][j] += mma2<TY>(a[0][i], b[0][j], a[1][i], b[1][j]);
         ++chain;
         int n = RAD;
 #pragma unroll
@@ -362,7 +372,7 @@ bool gemm_float_aligned(const FloatMM &f) {
 }
 
 // The tile kernels, from one 64 x 64 tile a CU on (f16 4096 x 4096: N = 200
-// 256 tiles, 37 us against 35 of the split, N = 256 37 against 38, N = 512 51
+// 256 tiles, 35 us against 35 of the split, N = 256 34 against 38, N = 512 49
 // against 77; 8192 x 4096 N = 64 128 tiles, 31 against 23). Up to 16 columns two a
 // CU (32768 x 4096: 46 against 56); f32, which would multiply 64 columns at an
 // eighth of the rate, above 32 columns only (4096 x 4096, N = 32: 106 against 23).
@@ -398,18 +408,21 @@ template <int TY, int B, int WM, int WN, int RAD, int LV, int D, int DX> static 
 
 template <int TY> static void launch_ty(const FloatMM &f, hipStream_t s) {
     if (gemm_float_tiled(f)) {
-        // by twos: the exactness above; it costs 64 x 64 tiles 5% (f16 4096 x 4096, N =
-        // 512: 53 against 51 us), and 128 x 128 tiles have no registers for it
-        const bool twos = TY == TLH_TYPE_F32 || (TY == TLH_TYPE_BF16 && f.K <= 1024);
-        // 128 x 128 tiles once there is one a CU (f16 8192 x 4096, N = 512: 71 us, with
+        // 128 x 128 tiles once there is one a CU (f16 8192 x 4096, N = 512: 67 us, with
         // 64 x 64 tiles 82; 4096 x 4096, N = 512, half as many: 65 against 44); f32 is
-        // bound by its MFMAs (8192 x 4096, N = 512: 320 against 292)
-        if constexpr (TY != TLH_TYPE_F16) {
-            if (twos) launch_tile<TY, 64, 2, 2, 2, 5, 4, 4>(f, s);
-        }
-        if constexpr (TY != TLH_TYPE_F32) {
-            if (!twos && tiles2(f, 128, 128) >= 256) launch_tile<TY, 128, 4, 2, 4, 3, 3, 2>(f, s);
-            else if (!twos) launch_tile<TY, 64, 2, 2, 4, 3, 4, 4>(f, s);
+        // bound by its MFMAs (8192 x 4096, N = 512: 320 against 292), and five levels
+        // have no registers there
+        const bool wide = tiles2(f, 128, 128) >= 256;
+        if constexpr (TY == TLH_TYPE_F16) {
+            if (wide) launch_tile<TY, 128, 4, 2, 8, 2, 3, 2>(f, s);
+            else launch_tile<TY, 64, 2, 2, 8, 2, 4, 4>(f, s);
+        } else if constexpr (TY == TLH_TYPE_BF16) {
+            // (by fours 8192 x 2048, N = 512 takes 42 us and 56 by twos)
+            if (f.K <= 1024) launch_tile<TY, 64, 2, 2, 2, 5, 4, 4>(f, s);
+            else if (wide) launch_tile<TY, 128, 4, 2, 4, 3, 3, 2>(f, s);
+            else launch_tile<TY, 64, 2, 2, 4, 3, 4, 4>(f, s);
+        } else {
+            launch_tile<TY, 64, 2, 2, 2, 5, 4, 4>(f, s);
         }
         return;
     }
