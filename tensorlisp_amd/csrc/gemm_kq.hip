@@ -312,12 +312,11 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
         commit(H0{}, r0);
         fetch(H0{}, sb0 + 1, r0);
         lds_barrier();
-        // Every 4 super-blocks the sums move to a second set (8 in long chunks), which
-        // keeps the chains of f32 additions short. Error against 64 bits, rms over rms,
-        // never / 8 / 4: q4_K 14336 x 14336, N = 48 1.10e-7 / 8.6e-8 / 8.5e-8, N = 512 (one
-        // chunk of 56) - / 8.8e-8 / 9.5e-8; 14336 x 4096, N = 64 7.6e-8 / 7.6e-8 / 7.2e-8; 4096 x
-        // 5632, 75 pairs an expert - / 7.85e-8 / 7.91e-8. In time, 8 and 4 are alike.
-        const int every = share > 20 ? 8 : 4;
+        // The sums move to a second set every few super-blocks (kq_unit.hpp). Error
+        // against 64 bits, rms over rms, in one chain / now: q4_K 14336 x 14336, N = 48
+        // 1.10e-7 / 8.5e-8; 14336 x 4096, N = 64 7.6e-8 / 7.2e-8. In time: q4_K
+        // 14336 x 4096, N = 512 107 -> 109 us.
+        const int every = kq_flush_every((int)(sb1 - sb0));
         auto flush = [&]() {
 #pragma unroll
             for (int j = 0; j < TN; ++j)
@@ -332,6 +331,7 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
         // us; 128 x 128 the other way round, N = 512: 126 against 110).
         constexpr bool NEST = BM == 64;
         int64_t sb = sb0;
+        int left = every;
         auto upto = [&](int64_t end) {
             for (; sb < end; ++sb) {
                 multiply(H0{});
@@ -344,7 +344,10 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
                 fetch(H0{}, sb + 2, r0);
                 if constexpr (!MIN) finalize();
                 if constexpr (!NEST) {
-                    if (((int)(sb - sb0) & (every - 1)) == every - 1) flush();
+                    if (--left == 0) {
+                        flush();
+                        left = every;
+                    }
                 }
                 lds_barrier();
             }

@@ -137,11 +137,12 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             kq_fetch<WT, H>(p + (int64_t)sb * SB, g, r);
         };
         kq_v4i S[P][NT];
-        // One column tile: every 4 super-blocks acc moves to tot, so that the f32 chains
-        // stay short (K = 8704 in one chunk, error against 64 bits: 1.16e-7 in one chain, 8.6e-8
+        // One column tile: acc moves to tot every few super-blocks (kq_unit.hpp; K = 8704 in one chunk, error against 64 bits: 1.16e-7 in one chain, 8.5e-8
         // now, a pair of its own 1.12e-7). Two have no registers for it and at most
         // 17 super-blocks a chunk (9.3e-8).
         constexpr bool FLUSH = NT == 1;
+        const int every = kq_flush_every(nsb);
+        int left = every;
         kq_v4f acc[NT], tot = {};
         auto multiply = [&](auto hc, int sb, const KqUnit<WT> &r) {
             constexpr int H = decltype(hc)::value;
@@ -214,9 +215,10 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             fetch(H1{}, sb + 2, u1, wrow, wnext, wnext2);
             if (++sb < nsb) {
                 if constexpr (FLUSH) {
-                    if ((sb & 3) == 0) {
+                    if (--left == 0) {
                         tot += acc[0];
                         acc[0] = (kq_v4f){};
+                        left = every;
                     }
                 }
                 return;
@@ -235,7 +237,7 @@ __global__ void __launch_bounds__(64 * KQS_WAVES) k_gemm_kqs(const MatmulArgs a,
             }
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[j] = (kq_v4f){};
-            if constexpr (FLUSH) tot = (kq_v4f){};
+            if constexpr (FLUSH) tot = (kq_v4f){}, left = every;
             sb = 0;
             b += workers;
             wrow = wnext;
